@@ -97,8 +97,13 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, bf16x2_t));
 }
 __device__ __forceinline__ float bf16_to_f32(uint32_t h) { return u2f(h << 16); }
-// IEEE binary16, round-to-nearest-even (v_cvt_f16_f32), subnormals kept.
-__device__ __forceinline__ uint32_t f32_to_f16(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
+// IEEE binary16, round-to-nearest-even (v_cvt_f16_f32), subnormals kept.  The empty asm statement
+// keeps the fp32 value a result of its own: hipcc otherwise folds the operation that made it and the
+// conversion into v_fma_mixlo_f16, which rounds once where ATen rounds to fp32 and then to fp16.
+__device__ __forceinline__ uint32_t f32_to_f16(float f) {
+    asm("" : "+v"(f));
+    return __builtin_bit_cast(uint16_t, (_Float16)f);
+}
 __device__ __forceinline__ float f16_to_f32(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }

@@ -69,6 +69,13 @@ __device__ __forceinline__ void words_to_f32(const uint32_t* w, float (&o)[4]) {
     }
 }
 
+// 4 values rounded to a 16-bit dtype, packed in order.
+template <int D>
+__device__ __forceinline__ u32x2 pack4_16(const float (&v)[4]) {
+    if constexpr (D == D_BF16) return u32x2{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
+    else return u32x2{f32_to_f16(v[0]) | (f32_to_f16(v[1]) << 16), f32_to_f16(v[2]) | (f32_to_f16(v[3]) << 16)};
+}
+
 template <int D>
 __device__ __forceinline__ void store_f32(uint64_t base, int64_t e, bool vec, const float (&v)[4]) {
     if constexpr (D == D_F32) {
@@ -80,19 +87,12 @@ __device__ __forceinline__ void store_f32(uint64_t base, int64_t e, bool vec, co
             for (int t = 0; t < 4; ++t) p[t] = v[t];
         }
     } else {
-        uint32_t h[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) h[t] = D == D_BF16 ? f32_to_bf16(v[t]) : f32_to_f16(v[t]);
         const gptr<uint16_t> p = gaddr<uint16_t>(base) + e;
         if (vec) {
-            if constexpr (D == D_BF16)
-                __builtin_nontemporal_store(u32x2{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])},
-                                            (gptr<u32x2>)p);
-            else
-                __builtin_nontemporal_store(u32x2{h[0] | (h[1] << 16), h[2] | (h[3] << 16)}, (gptr<u32x2>)p);
+            __builtin_nontemporal_store(pack4_16<D>(v), (gptr<u32x2>)p);
         } else {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) p[t] = (uint16_t)h[t];
+            for (int t = 0; t < 4; ++t) p[t] = (uint16_t)(D == D_BF16 ? f32_to_bf16(v[t]) : f32_to_f16(v[t]));
         }
     }
 }
@@ -263,15 +263,17 @@ __device__ __forceinline__ void decay4(const aw4_tensor& T, const float (&p)[4],
 // Tiles of tensors whose numel is a multiple of 128 (block layout)
 // ---------------------------------------------------------------------------
 
+constexpr bool is_16bit(int d) { return d == D_BF16 || d == D_F16; }
+
 // Whether a kernel moves parts of a tile between memory and its lanes through LDS: the specialised
-// bf16 kernels of the recipes (not the read-back or lookahead m2 ones).  Their lanes own 4 values
+// 16-bit kernels of the recipes (not the read-back or lookahead m2 ones).  Their lanes own 4 values
 // of a quarter, 8 bytes, so that direct accesses touch half of each 128-byte line per instruction
 // and the code words come in 2-byte loads.  Instead each lane loads one 8-byte piece of the tile's
 // codes and stores the 16-byte pieces of updated parameters 64 h + 8 j .. + 7 of its block, and
 // codes_to_lanes / params_to_memory rearrange them in LDS.  (Loading the gradients and
 // parameters the same way measured no faster, for 6 more registers.)
 constexpr bool lds_tile_io(int m1k, int m2k, int d) {
-    return d == D_BF16 && kind_of(m1k) != K_ANY && kind_of(m2k) != K_ANY && kind_of(m2k) != K_LA &&
+    return is_16bit(d) && kind_of(m1k) != K_ANY && kind_of(m2k) != K_ANY && kind_of(m2k) != K_LA &&
            (flags_of(m2k) & AW4_MOMENT_SAMPLED_READ) == 0;
 }
 // Whether a kernel loads its code bytes as one 8-byte piece per lane (codes_to_lanes): the
@@ -568,8 +570,7 @@ __device__ __forceinline__ void update_quarter(const aw4_tensor& T, int q, const
             else store_f32<D_F16>(T.param, e, vec, p);
         } else if constexpr (lds_tile_io(M1K, M2K, D)) {
             // the 8-byte piece into the tile's parameter image (params_to_memory stores it)
-            *(u32x2*)(p_img + image_column(tl.grp, 4 * q + (tl.j >> 1)) + 8u * (uint32_t)(tl.j & 1)) =
-                u32x2{f32x2_to_bf16x2(p[0], p[1]), f32x2_to_bf16x2(p[2], p[3])};
+            *(u32x2*)(p_img + image_column(tl.grp, 4 * q + (tl.j >> 1)) + 8u * (uint32_t)(tl.j & 1)) = pack4_16<D>(p);
         } else {
             store_f32<D>(tile_values<D>(T.param, tl.blk0), off, true, p);
         }
@@ -773,7 +774,7 @@ __device__ __forceinline__ bool values_only(const aw4_tensor& T) {
 // Tile order: grid order (wave w takes tiles w, w + W, ...) or consecutive tiles per wave
 // (w * K .. w * K + K - 1).  Prefetch: the next tile's loads are issued during the second
 // moment's encode.  Both keep the in-flight tiles of a memory-bound kernel adjacent and
-// its loads early.  The bf16 update-SR kernels, bound by their instruction issue, take
+// its loads early.  The 16-bit update-SR kernels, bound by their instruction issue, take
 // consecutive tiles (grid order cost them 2% at twelve tiles per wave, for its per-tile tensor
 // search).  The generic kernel (run-time kinds and dtype) has the register pressure of every
 // variant at once and loads each tile when it starts it.
@@ -789,7 +790,7 @@ constexpr bool prefetch_next_tile(int m1k, int m2k, int d) {
     return kind_of(m1k) != K_ANY && kind_of(m2k) != K_ANY && d != D_ANY && !research_kernel(m2k);
 }
 constexpr bool tile_order_grid(int m1k, int m2k, int d) {
-    return prefetch_next_tile(m1k, m2k, d) && !(kind_of(m2k) == K_USR && d == D_BF16);
+    return prefetch_next_tile(m1k, m2k, d) && !(kind_of(m2k) == K_USR && is_16bit(d));
 }
 // Update-SR kernels stage the new second moments in LDS (M2Staged) so that the prefetched
 // inputs fit in the registers of four waves per SIMD.

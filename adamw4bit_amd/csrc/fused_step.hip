@@ -293,12 +293,18 @@ struct KernelVariant {
 #define AW4_VARIANT_ILP(M1, M2, D) {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, nullptr}
 #define AW4_VARIANT_ILP_I4W(M1, M2, D) \
     {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, (const void*)&step_kernel_inline_4w<M1, M2, D>}
+// The fp16 recipes are bound as the bf16 ones are (memory for round-to-nearest, issue for update-SR)
+// and take the same tiles; before they had instances they ran the generic kernel, bound by its two
+// waves per SIMD: one Llama-3-8B layer (218M values) under ZE-EDEN 1,299 us there, 391-394 us here
+// (4.5 TB/s).  The fp16 update-SR ones spill under the max-ilp scheduler and keep the default one.
 const KernelVariant kVariants[] = {
     AW4_VARIANT_I4W(kRtn, kRtnEden, D_F32),       AW4_VARIANT_ILP_I4W(kRtn, kUsrGuarded, D_F32),
     AW4_VARIANT_I4W(kRtn, kRtnEden, D_BF16),      AW4_VARIANT_ILP_I4W(kRtn, kUsrGuarded, D_BF16),
     AW4_VARIANT(kSsrGuarded, kUsrGuarded, D_F32), AW4_VARIANT_ILP(kSsrGuarded, kUsrGuarded, D_BF16),
     AW4_VARIANT(kRtn, kFp32, D_F32),              AW4_VARIANT(kRtn, kFp32, D_BF16),
     AW4_VARIANT(kRtn, kUsrGuardedEden, D_F32),    AW4_VARIANT_ILP(kRtn, kUsrGuardedEden, D_BF16),
+    AW4_VARIANT_4W(kRtn, kRtnEden, D_F16),        AW4_VARIANT_4W(kRtn, kUsrGuarded, D_F16),
+    AW4_VARIANT_4W(kSsrGuarded, kUsrGuarded, D_F16),
     AW4_VARIANT(kRtn, kUsrRead, D_F32),           AW4_VARIANT(kRtn, kUsrReadEden, D_F32),
     AW4_VARIANT(kRtn, kLaStore, D_F32),           AW4_VARIANT_3W(kRtn, kLaPending, D_F32),
     AW4_VARIANT_2W(K_ANY, kAnyResearch, D_ANY),
@@ -693,7 +699,7 @@ struct LaunchGroup {
 
 // Split a step's tensors into launches: tensors that share a specialised kernel and its
 // tables form one launch each; fp32-state tensors join a specialised launch of their
-// dtype; everything else (other scheme mixes, fp16, mixed dtypes) runs in one launch of
+// dtype; everything else (other scheme mixes, float64, mixed dtypes) runs in one launch of
 // the generic kernel.  A recipe's table is one launch.
 std::vector<LaunchGroup> plan_launches(const aw4_tensor* ts, int32_t count) {
     std::vector<LaunchGroup> groups;
@@ -870,7 +876,7 @@ int large_tiles_per_wave(int variant, int64_t per_cu) {
     if (variant < kNumSpecialised) {
         const KernelVariant& kv = kVariants[variant];
         if (tile_order_grid(kv.m1, kv.m2, kv.dtype)) return 3;
-        if ((kind_of(kv.m2) == K_USR && kv.dtype == AW4_BF16) || research_kernel(kv.m2))
+        if ((kind_of(kv.m2) == K_USR && is_16bit(kv.dtype)) || research_kernel(kv.m2))
             return (int)std::max<int64_t>(kTilesPerWave, std::min<int64_t>(12, per_cu / 128));
     }
     return kTilesPerWave;
