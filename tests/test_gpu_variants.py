@@ -31,3 +31,24 @@ def test_fp16_recipe_kernels_match_oracle(m1, m2, eden):
                                         use_eden_m2=eden, quant_rng_seed=3, optimized=True)
     out = run_pair(make, SHAPES, torch.float16, 3, seed=3, zero_block_frac=0.02, grad_fn=fp16_safe)
     compare_pair(*out, f"fp16 {m1}/{m2}", steps=3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m1,m2", [("nf4", "dyn4_nz"), ("sdyn4", "lin4_nz"), ("nf4", "dyn4")])
+def test_round_to_nearest_pairs_match_oracle(m1, m2, dtype):
+    """Round-to-nearest first and second moments without EDEN: the optimized step's pairs of them."""
+    log(f"round-to-nearest {m1} / {m2} {dtype} x 3 steps")
+    make = lambda ps: aw.QuantizedAdamW(ps, lr=1e-3, weight_decay=0.1, m1_quant_scheme=m1, m2_quant_scheme=m2,  # noqa: E731
+                                        optimized=True)
+    out = run_pair(make, SHAPES, dtype, 3, seed=None, zero_block_frac=0.02, grad_fn=fp16_safe)
+    compare_pair(*out, f"{m1}/{m2} {dtype}", steps=3)
+
+
+@pytest.mark.parametrize("m2,eden", [("fp32", False), ("dyn4_upd_sr_fp32read", True)])
+def test_fp16_ablations_match_oracle(m2, eden):
+    """fp16 with an fp32 second moment, and with EDEN on the update-SR one."""
+    log(f"fp16 nf4 / {m2} eden={eden} x 3 steps")
+    make = lambda ps: aw.QuantizedAdamW(ps, lr=1e-3, weight_decay=0.1, m1_quant_scheme="nf4", m2_quant_scheme=m2,  # noqa: E731
+                                        use_eden_m2=eden, quant_rng_seed=3, optimized=True)
+    out = run_pair(make, SHAPES, torch.float16, 3, seed=3, zero_block_frac=0.02, grad_fn=fp16_safe)
+    compare_pair(*out, f"fp16 nf4/{m2}", steps=3)
