@@ -945,4 +945,98 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
     }
 }
 
+// ---------------------------------------------------------------------------
+// Launches of fp32-state tensors only
+// ---------------------------------------------------------------------------
+
+// n (1..4) values at element e as fp32: one vector access for a whole quad, single loads for the last
+// quad of a tensor.
+template <int D>
+__device__ __forceinline__ void load_quad(const aw4_tensor& T, uint64_t base, int64_t e, int n, bool vec, float (&o)[4]) {
+    if (n == 4) {
+        uint32_t w[4];
+        load_words<D>(base, e, vec, w);
+        words_to_f32<D>(w, o);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[t] = t < n ? load_value<D>(T, base, D, e + t) : 0.0f;
+    }
+}
+
+template <int D>
+__device__ __forceinline__ void store_quad(uint64_t base, int64_t e, int n, bool vec, const float (&v)[4]) {
+    if (n == 4) {
+        store_f32<D>(base, e, vec, v);
+    } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (t >= n) continue;
+            if constexpr (D == D_F32) gaddr<float>(base)[e + t] = v[t];
+            else gaddr<uint16_t>(base)[e + t] = (uint16_t)(D == D_BF16 ? f32_to_bf16(v[t]) : f32_to_f16(v[t]));
+        }
+    }
+}
+
+// A lane's four quads (values e0 + 32 q + 0..3) of one tile, as step_tile_values takes them, but loaded
+// together before the first store.  Every access except the last quad of a tensor is a vector of 4
+// values (the host aligns fp32 state to 16 bytes; parameters and gradients have the row's flag).
+// kWhole: the tile lies inside the tensor, no quad is cut.
+template <int D, bool kWhole>
+__device__ __forceinline__ void step_value_quads(const aw4_tensor& T, int64_t e0) {
+    const bool vec = (T.flags & AW4_TENSOR_VEC_ALIGNED) != 0;
+    const bool large1 = (T.flags & AW4_TENSOR_LERP1_LARGE) != 0, large2 = (T.flags & AW4_TENSOR_LERP2_LARGE) != 0;
+    float g[4][4], p[4][4], a[4][4], b[4][4];
+    int n[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int64_t e = e0 + 32 * q;
+        n[q] = kWhole ? 4 : (int)min((int64_t)4, T.numel - e);
+        if (n[q] <= 0) continue;
+        load_quad<D>(T, T.grad, e, n[q], vec, g[q]);
+        load_quad<D>(T, T.param, e, n[q], vec, p[q]);
+        load_quad<D_F32>(T, T.m1.values, e, n[q], true, a[q]);
+        load_quad<D_F32>(T, T.m2.values, e, n[q], true, b[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int64_t e = e0 + 32 * q;
+        if (n[q] <= 0) continue;
+        clip_grads<D>(T, g[q], 4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float gg = g[q][t] * g[q][t];
+            a[q][t] = __builtin_fmaf(T.w1, g[q][t] - a[q][t], large1 ? g[q][t] : a[q][t]);
+            b[q][t] = __builtin_fmaf(T.w2, gg - b[q][t], large2 ? gg : b[q][t]);
+            p[q][t] = param_update<D>(T, p[q][t], a[q][t], b[q][t]);
+        }
+        store_quad<D>(T.param, e, n[q], vec, p[q]);
+        store_quad<D_F32>(T.m1.values, e, n[q], true, a[q]);
+        store_quad<D_F32>(T.m2.values, e, n[q], true, b[q]);
+    }
+}
+
+// A launch of fp32-state tensors only (28 bytes a value in fp32, memory bound): no codec, so no LDS
+// tables, 84 VGPRs (six waves per SIMD), and each wave has its tile's 16 KB of loads in flight at once.
+// One tile per wave (no table to share between tiles).  A 201 MB fp32 set of odd sizes under ZIP-SR took
+// 69-71 us a step when these tiles went value by value inside the block kernel, 44 us here (4.5 TB/s);
+// a 306 MB fp16 one 357 -> 71 us, a 488 MB bf16 one 346 -> 98 us.
+template <int D>
+__device__ __forceinline__ void run_value_tiles(const StepHeader* hdr) {
+    const aw4_tensor* tensors = (const aw4_tensor*)(hdr + 1);
+    const int count = hdr->count;
+    const int64_t* tile_start = (const int64_t*)(tensors + count);
+    const int lane = threadIdx.x & 63;
+    const int64_t waves = (int64_t)gridDim.x * kWavesPerGroup;
+    int64_t tile = (int64_t)blockIdx.x * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int ti = 0;
+    for (int64_t k = 0; k < hdr->tiles_per_wave && tile < hdr->total_tiles; ++k, tile += waves) {
+        ti = tensor_of(tile_start, ti, count, tile);
+        const aw4_tensor& T = tensors[ti];
+        const int64_t e_tile = (tile - tile_start[ti]) * kWaveTile;
+        const int64_t e0 = e_tile + (lane >> 3) * kBlock + 4 * (lane & 7);
+        if (e_tile + kWaveTile <= T.numel) step_value_quads<D, true>(T, e0);
+        else step_value_quads<D, false>(T, e0);
+    }
+}
+
 }  // namespace aw4

@@ -220,6 +220,20 @@ step_kernel_inline_4w(const InlineArgs a) {
     step_body_inline<M1K, M2K, D>(a);
 }
 
+// A launch of fp32-state tensors only (run_value_tiles).
+template <int D>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+values_kernel(const StepHeader* __restrict__ hdr, const Tables* __restrict__) {
+    run_value_tiles<D>(hdr);
+}
+
+template <int D>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+values_kernel_inline(const InlineArgs a) {
+    run_value_tiles<D>(
+        (const StepHeader*)((const char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineArgs, table)));
+}
+
 }  // namespace
 
 // The four-wave update-SR kernels (ZIP-SR's fp32 and bf16 steps, the bf16 nf4_sr head and
@@ -294,6 +308,9 @@ struct KernelVariant {
 #define AW4_VARIANT_ILP(M1, M2, D) {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, nullptr}
 #define AW4_VARIANT_ILP_I4W(M1, M2, D) \
     {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, (const void*)&step_kernel_inline_4w<M1, M2, D>}
+// launches of fp32-state tensors of one dtype
+#define AW4_VARIANT_VALUES(D) \
+    {kFp32, kFp32, D, (const void*)&values_kernel<D>, (const void*)&values_kernel_inline<D>}
 // The fp16 recipes are bound as the bf16 ones are (memory for round-to-nearest, issue for update-SR)
 // and take the same tiles; before they had instances they ran the generic kernel, bound by its two
 // waves per SIMD: one Llama-3-8B layer (218M values) under ZE-EDEN 1,299 us there, 391-394 us here
@@ -311,12 +328,14 @@ const KernelVariant kVariants[] = {
     AW4_VARIANT(kRtn, kFp32, D_F16),              AW4_VARIANT_4W(kRtn, kUsrGuardedEden, D_F16),
     AW4_VARIANT_4W(kRtn, kRtn, D_F32),            AW4_VARIANT_4W(kRtn, kRtn, D_BF16),
     AW4_VARIANT_4W(kRtn, kRtn, D_F16),
+    AW4_VARIANT_VALUES(D_F32), AW4_VARIANT_VALUES(D_BF16), AW4_VARIANT_VALUES(D_F16),
     AW4_VARIANT(kRtn, kUsrRead, D_F32),           AW4_VARIANT(kRtn, kUsrReadEden, D_F32),
     AW4_VARIANT(kRtn, kLaStore, D_F32),           AW4_VARIANT_3W(kRtn, kLaPending, D_F32),
     AW4_VARIANT_2W(K_ANY, kAnyResearch, D_ANY),
     AW4_VARIANT(K_ANY, K_ANY, D_ANY),
 };
 #undef AW4_VARIANT
+#undef AW4_VARIANT_VALUES
 #undef AW4_VARIANT_4W
 #undef AW4_VARIANT_2W
 #undef AW4_VARIANT_3W
@@ -703,9 +722,64 @@ struct LaunchGroup {
     std::vector<int> members;
 };
 
+// fp32-state tensors of one dtype join the step's first launch of that dtype or take one of their own
+// (values_kernel).  Beside blocks a tile of them goes value by value, 10-20 us for its wave, at nobody's
+// expense while the launch has waves to spare; their own launch is faster per tile and costs about 1 us
+// (3 us of host time for a staged table) and a boundary on the stream.  Measured, us a step joined /
+// own, one block tensor and fp32-state tiles, ZIP-SR fp32 and bf16:
+//   1024^2 and 16-512 tiles: 15.9-16.2 / 17.1 and 15.8-16.9 / 17.1; 1024 tiles: 17.1 / 17.2 and
+//     17.4 / 17.5; 2048: 27.6 / 20.6 and 24.2 / 19.6; 4096: 47.6 / 30.1 and 44.2 / 29.9;
+//   8 tiles, which end the launch: 2048 x 3072 (24 tiles per CU, 2 fp32-state tiles) 25.5 / 30.0 and
+//     24.6 / 30.2; 2048 x 4096 (32) 37.9 / 32.3 and 41.7 / 32.2; 4096^2 (64) 53.3 / 54.5 and
+//     67.9 / 48.8 (a wave of consecutive tiles takes several of them); 14336 x 4096 157.6 / 158.7 and
+//     144.8 / 133.2;
+//   4096^2 and 16 tiles: 64.1 / 53.9 and 78.2 / 48.7.
+constexpr int64_t kValuesLaunchTiles = 1024;  // own launch from this many fp32-state tiles on
+constexpr int64_t kValuesBlockTiles = 8192;   // beside this many block tiles (32 per CU): own launch
+constexpr int64_t kValuesFewTiles = 16;       // ... unless they are fewer than this and in grid order
+
+bool values_variant(const KernelVariant& kv) { return kv.m1 == kFp32 && kv.m2 == kFp32; }
+
+int64_t tiles_of(const aw4_tensor* ts, const std::vector<int>& members) {
+    int64_t n = 0;
+    for (int i : members) n += (ts[i].numel + kWaveTile - 1) / kWaveTile;
+    return n;
+}
+
+void plan_values(const aw4_tensor* ts, const std::vector<int>& values, std::vector<LaunchGroup>& groups,
+                 LaunchGroup& generic) {
+    const size_t block_groups = groups.size();
+    for (int dtype : {AW4_F32, AW4_BF16, AW4_F16, AW4_F64}) {
+        std::vector<int> of;
+        for (int i : values)
+            if (ts[i].param_dtype == dtype) of.push_back(i);
+        if (of.empty()) continue;
+        int own = -1;  // this dtype's values_kernel (none for float64, which joins the generic launch)
+        for (int k = 0; k < kNumSpecialised; ++k)
+            if (kVariants[k].dtype == dtype && values_variant(kVariants[k])) own = k;
+        LaunchGroup* g = nullptr;
+        for (size_t k = 0; k < block_groups && !g; ++k)
+            if (kVariants[groups[k].variant].dtype == dtype) g = &groups[k];
+        if (!g && (own < 0 || !generic.members.empty())) g = &generic;
+        if (g && own >= 0) {
+            const KernelVariant& kv = kVariants[g->variant];
+            const int64_t tiles = tiles_of(ts, of);
+            const bool large = tiles_of(ts, g->members) >= kValuesBlockTiles &&
+                               (tiles >= kValuesFewTiles || !tile_order_grid(kv.m1, kv.m2, kv.dtype));
+            if (tiles >= kValuesLaunchTiles || large) g = nullptr;
+        }
+        if (!g) {
+            groups.emplace_back();
+            g = &groups.back();
+            g->variant = own;
+        }
+        g->members.insert(g->members.end(), of.begin(), of.end());
+    }
+}
+
 // Split a step's tensors into launches: tensors that share a specialised kernel and its
-// tables form one launch each; fp32-state tensors join a specialised launch of their
-// dtype; everything else (other scheme mixes, float64, mixed dtypes) runs in one launch of
+// tables form one launch each; fp32-state tensors join one of their dtype or form their own
+// (plan_values); everything else (other scheme mixes, float64, mixed dtypes) runs in one launch of
 // the generic kernel.  A recipe's table is one launch.
 std::vector<LaunchGroup> plan_launches(const aw4_tensor* ts, int32_t count) {
     std::vector<LaunchGroup> groups;
@@ -750,21 +824,7 @@ std::vector<LaunchGroup> plan_launches(const aw4_tensor* ts, int32_t count) {
         }
         g->members.push_back(i);
     }
-    for (int i : values) {
-        LaunchGroup* g = nullptr;
-        for (LaunchGroup& c : groups)
-            if (kVariants[c.variant].dtype == ts[i].param_dtype) { g = &c; break; }
-        if (!g && !generic.members.empty()) g = &generic;
-        if (!g) {
-            for (int k = 0; k < kNumSpecialised && !g; ++k) {
-                if (kVariants[k].dtype != ts[i].param_dtype) continue;
-                groups.emplace_back();
-                g = &groups.back();
-                g->variant = k;
-            }
-        }
-        (g ? g : &generic)->members.push_back(i);
-    }
+    plan_values(ts, values, groups, generic);
     if (!research.members.empty()) groups.push_back(std::move(research));
     if (!generic.members.empty()) groups.push_back(std::move(generic));
     for (LaunchGroup& g : groups) std::sort(g.members.begin(), g.members.end());
@@ -881,6 +941,7 @@ int prepare_step(const aw4_tensor* tensors, int32_t count, StepLaunch& sl) {
 int large_tiles_per_wave(int variant, int64_t per_cu) {
     if (variant < kNumSpecialised) {
         const KernelVariant& kv = kVariants[variant];
+        if (values_variant(kv)) return 1;
         if (tile_order_grid(kv.m1, kv.m2, kv.dtype)) return 3;
         if ((kind_of(kv.m2) == K_USR && is_16bit(kv.dtype)) || research_kernel(kv.m2))
             return (int)std::max<int64_t>(kTilesPerWave, std::min<int64_t>(12, per_cu / 128));
@@ -918,7 +979,8 @@ int fill_step_tables(const aw4_tensor* tensors, StepLaunch& sl, int num_cus, voi
         // least 1.  Measured on one 4096^2 ZIP-SR tensor (64 tiles per CU): 4 tiles per wave
         // 52.1-52.2 us, 2 52.7-52.9, 3 56.4-56.6, 1 57.1-57.3; one 1024^2 tensor (4 per CU): 1.
         const int64_t per_cu = acc / (int64_t)num_cus;
-        const int tiles_per_wave = per_cu >= 128 ? large_tiles_per_wave(lg.variant, per_cu)
+        const int tiles_per_wave = per_cu >= 128 || values_variant(kVariants[lg.variant])
+                                       ? large_tiles_per_wave(lg.variant, per_cu)
                                                  : (int)std::max<int64_t>(1, std::min<int64_t>(4, per_cu / 16));
         const int64_t waves = (acc + tiles_per_wave - 1) / tiles_per_wave;
         sl.grid[g] = (waves + kWavesPerGroup - 1) / kWavesPerGroup;

@@ -52,3 +52,48 @@ def test_fp16_ablations_match_oracle(m2, eden):
                                         use_eden_m2=eden, quant_rng_seed=3, optimized=True)
     out = run_pair(make, SHAPES, torch.float16, 3, seed=3, zero_block_frac=0.02, grad_fn=fp16_safe)
     compare_pair(*out, f"fp16 nf4/{m2}", steps=3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shapes", [[(1030, 1021), (1, 3), (1024,), (4,), (5,), (513, 2047)],  # a launch of their own
+                                    [(1030, 1021), (64, 128), (1024,), (2049, 511)],             # beside a block launch
+                                    [(3,), (1000,)]])                                           # few, and nothing else
+@pytest.mark.parametrize("betas", [(0.9, 0.95), (0.4, 0.45)])
+def test_fp32_state_launches_match_oracle(shapes, dtype, betas):
+    """fp32-state tensors in launches of their own: whole and cut tiles, the last quad of 1 to 3 values,
+    both lerp forms."""
+    log(f"fp32-state launches {dtype} {betas} {shapes}")
+    make = lambda ps: aw.ZIPSRAdamW4Bit(ps, lr=1e-3, betas=betas, weight_decay=0.1, quant_rng_seed=5, optimized=True)  # noqa: E731
+    out = run_pair(make, shapes, dtype, 2, seed=5, grad_fn=fp16_safe)
+    compare_pair(*out, f"fp32 state {dtype}", steps=2)
+
+
+def test_fp32_state_launch_with_misaligned_and_clipped_gradients():
+    """Gradients and parameters off a 16-byte boundary (single accesses), clipped in the same step, against
+    aligned copies of them stepped the same way."""
+    gen = torch.Generator().manual_seed(2)
+    n = 1025 * 1023
+    init, grad = torch.randn(n, generator=gen) * 0.02, torch.randn(n, generator=gen)
+    got = []
+    for shift in (0, 1):
+        p = torch.nn.Parameter(torch.zeros(n + 4, device=H.DEVICE)[shift:shift + n].copy_(init))
+        p.grad = torch.zeros(n + 4, device=H.DEVICE)[shift:shift + n].copy_(grad)
+        assert (p.data_ptr() % 16 == 0) == (shift == 0)
+        opt = aw.ZEEDENAdamW4Bit([p], optimized=True)
+        for _ in range(2):
+            opt.clip_grad_norm_(1.0)
+            opt.step()
+        got.append((p.detach().cpu(), opt.state[p]["m1"].cpu(), opt.state[p]["m2"].cpu()))
+    for a, b in zip(*got):
+        assert torch.equal(H.bits(a), H.bits(b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_fp32_state_beside_a_large_block_launch(dtype):
+    """A block launch of 32 tiles per CU and more, with fewer and more fp32-state tiles than the few that
+    join it in grid order."""
+    for extra in ([(4095,)], [(4095,)] * 5):
+        log(f"fp32-state tiles beside 2048x4096 {dtype} {len(extra)}")
+        make = lambda ps: aw.ZIPSRAdamW4Bit(ps, lr=1e-3, weight_decay=0.1, quant_rng_seed=5, optimized=True)  # noqa: E731
+        out = run_pair(make, [(2048, 4096)] + extra, dtype, 2, seed=5)
+        compare_pair(*out, f"fp32 state beside blocks {dtype}", steps=2)
