@@ -348,57 +348,106 @@ constexpr int kGenericVariant = kNumVariants - 1;
 constexpr int kResearchVariant = kNumVariants - 2;  // generic, for read-back and lookahead m2
 constexpr int kNumSpecialised = kResearchVariant;
 
-// Stand-alone codec kernels (one wave tile per wave, grid-stride).
+// Stand-alone codec kernels.  They stream (encode reads 4 bytes and writes 0.53 a value, decode the
+// reverse), so a workgroup's LDS holds only the tables its one moment needs (8 KB of tables and the four
+// waves' scratch to encode, 2 KB to decode; all codebooks' tables are 36 KB and left three workgroups to
+// a CU), and the grid covers every tile at kCodecTiles per wave, which share the table fill.
+// Measured, nf4, us encode / decode of 2^24 values: 28 / 28 with all tables and a grid of eight
+// workgroups per CU, 14.9 / 13.4 so (5.1 / 5.7 TB/s); 2^27 values 112 / 124 us (5.4 / 4.9 TB/s).
+// Encoding nf4_sr is bound by its draws (26.7 us).
+constexpr int kCodecTiles = 4;
+
+// Encode tables of the codebook a moment uses, and the waves' scratch.
+struct LdsEncode {
+    float cb[16];
+    UsrPair usr[kPairs];
+    PairEntry pairs[kPairs];
+    LutEntry lut[AW4_LUT_ENTRIES];
+    WaveScratch scratch[kWavesPerGroup];
+
+    __device__ void load(const Tables* g, int codebook, int lut_id) {
+        if (threadIdx.x < 16) cb[threadIdx.x] = g->codebook[codebook][threadIdx.x];
+        if (threadIdx.x < kPairs) {
+            usr[threadIdx.x] = g->usr[codebook][threadIdx.x];
+            pairs[threadIdx.x] = g->pairs[codebook][threadIdx.x];
+        }
+        if (threadIdx.x < AW4_LUT_ENTRIES) lut[threadIdx.x] = g->lut[lut_id][threadIdx.x];
+        __syncthreads();
+    }
+};
+static_assert(AW4_LUT_ENTRIES <= kThreads, "one thread per lookup entry");
+
+// KIND: the moment's rounding (its flags are read at run time).  Wave w of W encodes tiles w, w + W, ...,
+// the next tile's values loaded while this one is encoded.
+template <int KIND>
 __global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restrict__ values, int64_t numel,
                                                             aw4_moment M, const Tables* __restrict__ tables) {
-    __shared__ LdsAll lds;
-    lds.load(tables, nullptr);
+    __shared__ LdsEncode lds;
     const int lane = threadIdx.x & 63;
     const int wslot = threadIdx.x >> 6;
     const int j = lane & 7, grp = lane >> 3;
     const int64_t nblocks = numel / kBlock;
     const int64_t tiles = (nblocks + kBlocksPerWave - 1) / kBlocksPerWave;
     const int64_t nwaves = (int64_t)gridDim.x * kWavesPerGroup;
-    const MomentTables L = lds.moment(M, 0);
-    for (int64_t tile = (int64_t)blockIdx.x * kWavesPerGroup + wslot; tile < tiles; tile += nwaves) {
-        const int64_t blk = tile * kBlocksPerWave + grp;
-        const bool active = blk < nblocks;
-        float m[16];
+    int64_t tile = (int64_t)blockIdx.x * kWavesPerGroup + __builtin_amdgcn_readfirstlane(wslot);
+    auto load = [&](int64_t t, float (&m)[16]) {
+        const int64_t blk = t * kBlocksPerWave + grp;
+        // a lane past the last block reads the tile's first block, which exists; nothing of it is stored
+        const float* v = values + (blk < nblocks ? blk : t * kBlocksPerWave) * kBlock + 4 * j;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (active) v = *(const float4*)(values + blk * kBlock + 32 * q + 4 * j);
-            m[4 * q] = v.x; m[4 * q + 1] = v.y; m[4 * q + 2] = v.z; m[4 * q + 3] = v.w;
+            const f32x4 x = *(gptr<const f32x4>)gaddr<const float>((uint64_t)(v + 32 * q));
+            m[4 * q] = x.x; m[4 * q + 1] = x.y; m[4 * q + 2] = x.z; m[4 * q + 3] = x.w;
         }
+    };
+    float next[16];
+    if (tile < tiles) load(tile, next);
+    lds.load(tables, M.codebook, lut_id_of(M.rounding, M.codebook, M.flags));
+    const MomentTables L{lds.cb, lds.pairs, nullptr, lds.lut, lds.usr};
+    while (tile < tiles) {
+        float m[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m[i] = next[i];
+        const int64_t blk0 = tile * kBlocksPerWave;
+        tile += nwaves;
+        if (tile < tiles) load(tile, next);
         // stand-alone encodes accept any sign (a first moment or a caller's values)
-        encode_block_any<false>(M, L, tile * kBlocksPerWave, grp, j, active, RegValues{m}, lds.scratch[wslot].block(grp));
+        encode_block<mspec(KIND, kFlagsAtRunTime), false>(M, L, blk0, grp, j, blk0 + grp < nblocks, RegValues{m},
+                                                          lds.scratch[wslot].block(grp));
     }
 }
 
+// Wave w of W decodes tiles w, w + W, ...; in a tile, load q of lane l is the two code bytes of values
+// 256 q + 4 l .. + 3, so a wave's loads and stores are contiguous (128 bytes and 1 KB).
 __global__ void __launch_bounds__(kThreads) dequantize_kernel(aw4_moment M, int64_t numel, float* __restrict__ out,
                                                               const Tables* __restrict__ tables) {
-    __shared__ LdsAll lds;
-    lds.load(tables, nullptr);
+    __shared__ float2 dec[256];
+    static_assert(kThreads == 256, "one thread per decode entry");
+    dec[threadIdx.x] = tables->dec[M.codebook][threadIdx.x];
+    __syncthreads();
     const int lane = threadIdx.x & 63;
-    const int wslot = threadIdx.x >> 6;
-    const int j = lane & 7, grp = lane >> 3;
-    const int64_t nblocks = numel / kBlock;
-    const int64_t tiles = (nblocks + kBlocksPerWave - 1) / kBlocksPerWave;
+    const int64_t tiles = (numel + kWaveTile - 1) / kWaveTile;
     const int64_t nwaves = (int64_t)gridDim.x * kWavesPerGroup;
-    const MomentTables L = lds.moment(M, 0);
-    for (int64_t tile = (int64_t)blockIdx.x * kWavesPerGroup + wslot; tile < tiles; tile += nwaves) {
-        const int64_t blk = tile * kBlocksPerWave + grp;
-        if (blk >= nblocks) continue;
+    const gptr<const uint8_t> codes = gaddr<const uint8_t>(M.codes);
+    const gptr<const float> scales = gaddr<const float>(M.scales);
+    for (int64_t tile = (int64_t)blockIdx.x * kWavesPerGroup + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+         tile < tiles; tile += nwaves) {
+        const int64_t e0 = tile * kWaveTile + 4 * lane;
         uint32_t w[4];
-        const gptr<const uint8_t> codes = gaddr<const uint8_t>(M.codes) + blk * (kBlock / 2) + 2 * j;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] = *(gptr<const uint16_t>)(codes + 16 * q);
-        const float scale = gaddr<const float>(M.scales)[blk];
+        float scale[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
+            const int64_t e = e0 + 256 * q;
+            const int64_t at = e < numel ? e : 4 * (lane & 31);  // past the end: the first block's, not stored
+            w[q] = *(gptr<const uint16_t>)(codes + at / 2);
+            scale[q] = scales[at / kBlock];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t e = e0 + 256 * q;
             float m[4];
-            decode4(L.dec, w[q], scale, m);
-            *(float4*)(out + blk * kBlock + 32 * q + 4 * j) = make_float4(m[0], m[1], m[2], m[3]);
+            decode4(dec, w[q], scale[q], m);
+            if (e < numel) *(gptr<f32x4>)gaddr<float>((uint64_t)(out + e)) = f32x4{m[0], m[1], m[2], m[3]};
         }
     }
 }
@@ -1085,6 +1134,15 @@ int upload_by_arguments(const void* src, size_t bytes, uint8_t* dst, hipStream_t
     return AW4_OK;
 }
 
+// Workgroups of a codec launch: kCodecTiles tiles per wave once that leaves every CU eight workgroups,
+// fewer below (the kernels' waves stride over whatever tiles the grid leaves).
+unsigned codec_groups(int64_t numel, int num_cus) {
+    const int64_t tiles = (numel + kWaveTile - 1) / kWaveTile;
+    const int64_t per_wave = std::max<int64_t>(1, std::min<int64_t>(kCodecTiles, tiles / (num_cus * 8 * kWavesPerGroup)));
+    const int64_t groups = (tiles + per_wave * kWavesPerGroup - 1) / (per_wave * kWavesPerGroup);
+    return (unsigned)std::min<int64_t>(groups, 0x7fffffff);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1180,11 +1238,10 @@ int aw4_quantize(const float* values, int64_t numel, const aw4_moment* m, void* 
     DeviceState* ds = nullptr;
     rc = device_state(&ds);
     if (rc) return rc;
-    const int64_t tiles = (numel / kBlock + kBlocksPerWave - 1) / kBlocksPerWave;
-    int64_t groups = (tiles + kWavesPerGroup - 1) / kWavesPerGroup;
-    if (groups > (int64_t)ds->num_cus * 8) groups = (int64_t)ds->num_cus * 8;
-    hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)groups), dim3(kThreads), 0, (hipStream_t)stream, values, numel,
-                       *m, (const Tables*)ds->tables);
+    auto kernel = m->rounding == AW4_ROUND_RTN ? quantize_kernel<K_RTN>
+                : m->rounding == AW4_ROUND_STATE_SR ? quantize_kernel<K_SSR> : quantize_kernel<K_USR>;
+    hipLaunchKernelGGL(kernel, dim3(codec_groups(numel, ds->num_cus)), dim3(kThreads), 0, (hipStream_t)stream, values, numel, *m,
+                       (const Tables*)ds->tables);
     AW4_HIP_CHECK(hipGetLastError());
     return AW4_OK;
 }
@@ -1202,11 +1259,8 @@ int aw4_dequantize(const aw4_moment* m, int64_t numel, float* out, void* stream)
     DeviceState* ds = nullptr;
     int rc = device_state(&ds);
     if (rc) return rc;
-    const int64_t tiles = (numel / kBlock + kBlocksPerWave - 1) / kBlocksPerWave;
-    int64_t groups = (tiles + kWavesPerGroup - 1) / kWavesPerGroup;
-    if (groups > (int64_t)ds->num_cus * 8) groups = (int64_t)ds->num_cus * 8;
-    hipLaunchKernelGGL(dequantize_kernel, dim3((unsigned)groups), dim3(kThreads), 0, (hipStream_t)stream, *m, numel,
-                       out, (const Tables*)ds->tables);
+    hipLaunchKernelGGL(dequantize_kernel, dim3(codec_groups(numel, ds->num_cus)), dim3(kThreads), 0,
+                       (hipStream_t)stream, *m, numel, out, (const Tables*)ds->tables);
     AW4_HIP_CHECK(hipGetLastError());
     return AW4_OK;
 }

@@ -9,8 +9,11 @@ import pytest
 import torch
 
 import adamw4bit_amd as aw
+from adamw4bit_amd import _lib
+from adamw4bit_amd import quantization as q
+from oracle import reference_step as ref
 from tests import gpu_helpers as H
-from tests.test_gpu_step import compare_pair, log, run_pair
+from tests.test_gpu_step import compare_pair, gpu_encode, log, moment_desc, run_pair, stream
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +100,27 @@ def test_fp32_state_beside_a_large_block_launch(dtype):
         make = lambda ps: aw.ZIPSRAdamW4Bit(ps, lr=1e-3, weight_decay=0.1, quant_rng_seed=5, optimized=True)  # noqa: E731
         out = run_pair(make, [(2048, 4096)] + extra, dtype, 2, seed=5)
         compare_pair(*out, f"fp32 state beside blocks {dtype}", steps=2)
+
+
+@pytest.mark.parametrize("blocks", [1, 7, 8, 9, 33, 8 * 4 * 256 * 8 + 5])
+@pytest.mark.parametrize("mode,eden", [("nf4", False), ("dyn4_nz", True), ("nf4_sr", False), ("dyn4_upd_sr_fp32read", False)])
+def test_codec_sizes_match_oracle(mode, eden, blocks):
+    """aw4_quantize and aw4_dequantize from one block to more tiles than a wave each: whole and cut tiles."""
+    log(f"codec {mode} {blocks} blocks")
+    gen = torch.Generator().manual_seed(blocks)
+    values = H.heavy_tailed((blocks, 128), gen).reshape(-1)
+    if mode.startswith("dyn4"):
+        values = values.square()
+    values[:128] = 0.0
+    draws = torch.rand(blocks, 128, generator=gen) if "sr" in mode else None
+    codes, scales = gpu_encode(values, mode, eden, True, draws)
+    expect, expect_scales = ref.encode(values, mode, eden=eden, draws=draws, usr_sqrt="cr")
+    assert torch.equal(q.unpack_4bit_codes(codes, numel=values.numel()), expect)
+    assert torch.equal(H.bits(scales), H.bits(expect_scales))
+    packed, sc = codes.to(H.DEVICE), scales.to(H.DEVICE)
+    out = torch.full((values.numel() + 64,), 7.0, device=H.DEVICE)
+    _lib.dequantize(moment_desc(mode, eden, True, packed, sc), values.numel(), out.data_ptr(), stream())
+    torch.cuda.synchronize()
+    levels = q.codebook_tensor(mode)
+    assert torch.equal(H.bits(out[:values.numel()]), H.bits(levels[expect.long()] * expect_scales.repeat_interleave(128)))
+    assert bool((out[values.numel():] == 7.0).all())
