@@ -3,8 +3,8 @@
 // run before every step (an HF Trainer with max_grad_norm=1.0,
 // examples/train_gpt_small.py:214), optionally of the gradients GradScaler.unscale_ would leave
 // (the loss scale's inverse applied in the same read).  One pass over the gradients: each
-// workgroup sums the squares of one segment of one gradient in float64; one wave per gradient
-// then combines its segments, and a single workgroup adds the per-gradient squares, both in a
+// workgroup sums the squares of one segment of one gradient in float64; the last workgroup of a
+// gradient then combines its segments, and the last of all adds the per-gradient squares, both in a
 // fixed order, with torch's rounding points (clip_grad.py _get_total_norm /
 // _clip_grads_with_norm_):
 //   g'     = grad_dtype(fp32(g * u))                   (unscaling: _amp_foreach_non_finite_check_and_unscale_)
@@ -22,23 +22,36 @@
 namespace aw4 {
 
 constexpr int kNormThreads = 256;
-constexpr int64_t kNormSegment = 1 << 18;  // gradient values per workgroup of the norm pass
+// Gradient values per workgroup of the norm pass: 2^13 (one batch of eight vector loads per thread) to
+// 2^18, the host's choice by the total (norm_segment_shift).
+constexpr int kNormShiftMin = 13, kNormShiftMax = 18;
+
+// One gradient of the pass (24 bytes: the rows of 156 gradients fit a launch's arguments).
+struct NormRow {
+    uint64_t grad;      // device address
+    int64_t numel;
+    int32_t seg_start;  // first of its segments
+    int32_t dtype;      // AW4_* of the gradient, with kNormVec where 4-value vector access is allowed
+};
+constexpr int kNormVec = 0x100;
 
 struct NormHeader {
     int32_t count;
     int32_t result_dtype;  // R
     float max_norm;
     int32_t unscale;       // nonzero: unscale by *inv_scale, and report found_inf
-    int64_t total_segments;
+    int32_t total_segments;
+    int32_t segment_shift;
     uint64_t partials;     // device address, double[total_segments]
     uint64_t norm_sq;      // device address, double[count]: norm_t^2 of each gradient
+    uint64_t tickets;      // device address, uint32[count + 1], zero before and after the launch
     uint64_t norm_out;     // device address, float
     uint64_t coef_out;     // device address, float
     uint64_t inv_scale;    // device address, float u (unscale)
     uint64_t nonfinite;    // device address, uint32[total_segments]: a segment holds a non-finite g (unscale)
     uint64_t found_out;    // device address, float found_inf (unscale)
 };
-// followed by aw4_tensor rows[count] and int64_t seg_start[count + 1]
+// followed by NormRow rows[count]
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
@@ -59,10 +72,10 @@ __device__ __forceinline__ double sq1(float f, float u, bool& bad) {
 
 // Sum of squares of 4 consecutive gradient values starting at element e (all in range).
 template <int G, bool kUnscale>
-__device__ __forceinline__ double sq4(const aw4_tensor& T, int64_t e, bool vec, float u, bool& bad) {
+__device__ __forceinline__ double sq4(uint64_t grad, int64_t e, bool vec, float u, bool& bad) {
     uint32_t w[4];
     float f[4];
-    load_words<G>(T.grad, e, vec, w);
+    load_words<G>(grad, e, vec, w);
     words_to_f32<G>(w, f);
     double s = 0.0;
 #pragma unroll
@@ -71,7 +84,7 @@ __device__ __forceinline__ double sq4(const aw4_tensor& T, int64_t e, bool vec, 
 }
 
 template <int G, bool kUnscale>
-__device__ __forceinline__ double segment_sum(const aw4_tensor& T, int64_t e0, int64_t e1, bool vec, float u,
+__device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t e1, bool vec, float u,
                                               bool& bad) {
     // Full groups of 4 values: thread i takes groups i, i + 256, ... (8 loads in flight per
     // thread: 4 KB per workgroup per load instruction).
@@ -81,18 +94,18 @@ __device__ __forceinline__ double segment_sum(const aw4_tensor& T, int64_t e0, i
     for (; k + 7 * kNormThreads < groups; k += 8 * kNormThreads) {
         double s[8];
 #pragma unroll
-        for (int v = 0; v < 8; ++v) s[v] = sq4<G, kUnscale>(T, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
+        for (int v = 0; v < 8; ++v) s[v] = sq4<G, kUnscale>(grad, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
 #pragma unroll
         for (int v = 0; v < 8; ++v) acc += s[v];
     }
-    for (; k < groups; k += kNormThreads) acc += sq4<G, kUnscale>(T, e0 + 4 * k, vec, u, bad);
+    for (; k < groups; k += kNormThreads) acc += sq4<G, kUnscale>(grad, e0 + 4 * k, vec, u, bad);
     // the tail of the tensor (fewer than 4 values)
     const int64_t tail = e0 + 4 * groups;
     if ((int64_t)threadIdx.x < e1 - tail) {
         float f;
-        if (G == D_F32) f = gaddr<const float>(T.grad)[tail + threadIdx.x];
+        if (G == D_F32) f = gaddr<const float>(grad)[tail + threadIdx.x];
         else {
-            const uint32_t h = gaddr<const uint16_t>(T.grad)[tail + threadIdx.x];
+            const uint32_t h = gaddr<const uint16_t>(grad)[tail + threadIdx.x];
             f = G == D_BF16 ? bf16_to_f32(h) : f16_to_f32(h);
         }
         acc += sq1<G, kUnscale>(f, u, bad);
@@ -100,85 +113,66 @@ __device__ __forceinline__ double segment_sum(const aw4_tensor& T, int64_t e0, i
     return acc;
 }
 
-// One workgroup per segment: the float64 sum of squares of values
-// [s * kNormSegment, min((s + 1) * kNormSegment, numel)) of one gradient -> partials[seg].
-__global__ void __launch_bounds__(kNormThreads) norm_partials_kernel(const NormHeader* hdr) {
-    const aw4_tensor* rows = (const aw4_tensor*)(hdr + 1);
-    const int count = hdr->count;
-    const int64_t* seg_start = (const int64_t*)(rows + count);
-    const int64_t seg = blockIdx.x;
-    const int t = tensor_of(seg_start, 0, count, seg);
-    const aw4_tensor& T = rows[t];
-    const int64_t e0 = (seg - seg_start[t]) * kNormSegment;
-    const int64_t e1 = min(e0 + kNormSegment, T.numel);
-    const bool vec = (T.flags & AW4_TENSOR_VEC_ALIGNED) != 0;
-    double acc;
-    bool bad = false;
-    if (hdr->unscale) {
-        const float u = *gaddr<const float>(hdr->inv_scale);
-        if (T.grad_dtype == D_F32) acc = segment_sum<D_F32, true>(T, e0, e1, vec, u, bad);
-        else if (T.grad_dtype == D_BF16) acc = segment_sum<D_BF16, true>(T, e0, e1, vec, u, bad);
-        else acc = segment_sum<D_F16, true>(T, e0, e1, vec, u, bad);
-    } else {
-        if (T.grad_dtype == D_F32) acc = segment_sum<D_F32, false>(T, e0, e1, vec, 1.0f, bad);
-        else if (T.grad_dtype == D_BF16) acc = segment_sum<D_BF16, false>(T, e0, e1, vec, 1.0f, bad);
-        else acc = segment_sum<D_F16, false>(T, e0, e1, vec, 1.0f, bad);
-    }
-    acc = wave_sum_f64(acc);
-    const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
-    __shared__ double wave_acc[kNormThreads / 64];
-    __shared__ uint32_t wave_bad_any[kNormThreads / 64];
-    if ((threadIdx.x & 63) == 0) {
-        wave_acc[threadIdx.x >> 6] = acc;
-        wave_bad_any[threadIdx.x >> 6] = wave_bad ? 1u : 0u;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = wave_acc[0];
-        uint32_t b = wave_bad_any[0];
-#pragma unroll
-        for (int w = 1; w < kNormThreads / 64; ++w) {
-            s += wave_acc[w];
-            b |= wave_bad_any[w];
-        }
-        gaddr<double>(hdr->partials)[seg] = s;
-        if (hdr->unscale) gaddr<uint32_t>(hdr->nonfinite)[seg] = b;
-    }
+// What one workgroup leaves for another goes through device-scope atomic accesses only (the XCDs' L2
+// caches are not coherent for plain ones within a launch): a store written through, complete when
+// draw_ticket's wait returns, then the ticket, and loads past the caches by whoever drew the last one.
+// A release and an acquire in their place would also write back and invalidate an L2 per workgroup, for
+// plain stores that none of them reads: 195 us a pass more for GPT-2-small, after a step's dirty lines.
+template <class T>
+__device__ __forceinline__ T agent_load(gptr<T> p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void agent_store(gptr<T> p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One wave per gradient t: norm_sq[t] = norm_t^2 from its segments (lanes stride over them).
-__global__ void __launch_bounds__(64) norm_tensor_kernel(const NormHeader* hdr) {
-    const aw4_tensor* rows = (const aw4_tensor*)(hdr + 1);
-    const int count = hdr->count;
-    const int64_t* seg_start = (const int64_t*)(rows + count);
-    const gptr<const double> partials = gaddr<const double>(hdr->partials);
-    const int t = blockIdx.x;
+__device__ __forceinline__ uint32_t draw_ticket(gptr<uint32_t> p) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keeps the order in the compiler
+    __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0): this thread's stores are complete
+    const uint32_t drawn = __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return drawn;
+}
+
+// The index of the gradient that holds a segment.
+__device__ __forceinline__ int norm_row_of(const NormRow* rows, int count, int seg) {
+    int lo = 0, hi = count - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (rows[mid].seg_start <= seg) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+// norm_t^2 of one gradient from its segments' sums (lanes stride over them): wave 0 of its last workgroup.
+__device__ __forceinline__ double norm_tensor_sq(const NormHeader* hdr, int first, int end, int dtype) {
+    const gptr<double> partials = gaddr<double>(hdr->partials);
     double s = 0.0;
-    for (int64_t k = seg_start[t] + threadIdx.x; k < seg_start[t + 1]; k += 64) s += partials[k];
+    for (int k = first + (int)threadIdx.x; k < end; k += 64) s += agent_load(partials + k);
     s = wave_sum_f64(s);
-    if (threadIdx.x == 0) {
-        const float norm_t = round_to_dtype((float)__builtin_sqrt(s), rows[t].grad_dtype);
-        gaddr<double>(hdr->norm_sq)[t] = (double)norm_t * (double)norm_t;  // exact
-    }
+    const float norm_t = round_to_dtype((float)__builtin_sqrt(s), dtype);
+    return (double)norm_t * (double)norm_t;  // exact
 }
 
-// One workgroup: thread i adds norm_sq[i], norm_sq[i + 256], ...; the sums of the 4 waves are
-// added in order; then the total norm and the coefficient.
-__global__ void __launch_bounds__(kNormThreads) norm_finish_kernel(const NormHeader* hdr) {
+// The total norm and the coefficient, by the whole of the launch's last workgroup: thread i adds
+// norm_sq[i], norm_sq[i + 256], ...; the sums of the 4 waves are added in order.
+__device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_sq, uint32_t* wave_bad_any) {
     const int count = hdr->count;
-    const gptr<const double> norm_sq = gaddr<const double>(hdr->norm_sq);
+    const gptr<double> norm_sq = gaddr<double>(hdr->norm_sq);
+    const gptr<uint32_t> tickets = gaddr<uint32_t>(hdr->tickets);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double sq = 0.0;
-    for (int t = threadIdx.x; t < count; t += kNormThreads) sq += norm_sq[t];
+    for (int t = threadIdx.x; t < count; t += kNormThreads) sq += agent_load(norm_sq + t);
+    for (int t = threadIdx.x; t <= count; t += kNormThreads) tickets[t] = 0;  // every workgroup has drawn its own
     sq = wave_sum_f64(sq);
     uint32_t bad = 0;
     if (hdr->unscale) {
-        const gptr<const uint32_t> nonfinite = gaddr<const uint32_t>(hdr->nonfinite);
-        for (int64_t k = threadIdx.x; k < hdr->total_segments; k += kNormThreads) bad |= nonfinite[k];
+        const gptr<uint32_t> nonfinite = gaddr<uint32_t>(hdr->nonfinite);
+        for (int k = threadIdx.x; k < hdr->total_segments; k += kNormThreads) bad |= agent_load(nonfinite + k);
     }
     const bool wave_bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
-    __shared__ double wave_sq[kNormThreads / 64];
-    __shared__ uint32_t wave_bad_any[kNormThreads / 64];
+    __syncthreads();  // the arrays' earlier contents have been read
     if (lane == 0) {
         wave_sq[wave] = sq;
         wave_bad_any[wave] = wave_bad ? 1u : 0u;
@@ -203,6 +197,83 @@ __global__ void __launch_bounds__(kNormThreads) norm_finish_kernel(const NormHea
         *gaddr<float>(hdr->norm_out) = total;
         *gaddr<float>(hdr->coef_out) = coef;
     }
+}
+
+// One workgroup per segment: the float64 sum of squares of its values -> partials[seg].  The workgroup
+// that draws a gradient's last ticket adds up that gradient's segments, and the one that then draws the
+// last gradient's ticket the whole (no workgroup waits for another; the sums' order is fixed, whichever
+// workgroups those are).  Bound by the read of the gradients; as three launches behind a staged table
+// (segments, gradients, total) the last two took 5 us each for GPT-2-small's 148 gradients, and longer
+// than the read for a small model's.  Clip and step: GPT-2-small 431 -> 428 us, a tiny GPT-2 (host bound)
+// 135 -> 127 us, 9 MB of bf16 gradients in seven tensors 82 -> 73 us.
+__device__ __forceinline__ void norm_body(const NormHeader* hdr) {
+    const NormRow* rows = (const NormRow*)(hdr + 1);
+    const int count = hdr->count;
+    const int seg = (int)blockIdx.x;
+    const int t = norm_row_of(rows, count, seg);
+    const NormRow& T = rows[t];
+    const int end = t + 1 < count ? rows[t + 1].seg_start : hdr->total_segments;
+    const int dtype = T.dtype & (kNormVec - 1);
+    const int64_t e0 = (int64_t)(seg - T.seg_start) << hdr->segment_shift;
+    const int64_t e1 = min(e0 + ((int64_t)1 << hdr->segment_shift), T.numel);
+    const bool vec = (T.dtype & kNormVec) != 0;
+    double acc;
+    bool bad = false;
+    if (hdr->unscale) {
+        const float u = *gaddr<const float>(hdr->inv_scale);
+        if (dtype == D_F32) acc = segment_sum<D_F32, true>(T.grad, e0, e1, vec, u, bad);
+        else if (dtype == D_BF16) acc = segment_sum<D_BF16, true>(T.grad, e0, e1, vec, u, bad);
+        else acc = segment_sum<D_F16, true>(T.grad, e0, e1, vec, u, bad);
+    } else {
+        if (dtype == D_F32) acc = segment_sum<D_F32, false>(T.grad, e0, e1, vec, 1.0f, bad);
+        else if (dtype == D_BF16) acc = segment_sum<D_BF16, false>(T.grad, e0, e1, vec, 1.0f, bad);
+        else acc = segment_sum<D_F16, false>(T.grad, e0, e1, vec, 1.0f, bad);
+    }
+    acc = wave_sum_f64(acc);
+    const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    __shared__ double wave_acc[kNormThreads / 64];
+    __shared__ uint32_t wave_bad_any[kNormThreads / 64];
+    __shared__ uint32_t last_of_gradient, last_of_all;  // this workgroup drew the last ticket
+    if ((threadIdx.x & 63) == 0) {
+        wave_acc[threadIdx.x >> 6] = acc;
+        wave_bad_any[threadIdx.x >> 6] = wave_bad ? 1u : 0u;
+    }
+    __syncthreads();
+    const gptr<uint32_t> tickets = gaddr<uint32_t>(hdr->tickets);
+    if (threadIdx.x == 0) {
+        double s = wave_acc[0];
+        uint32_t b = wave_bad_any[0];
+#pragma unroll
+        for (int w = 1; w < kNormThreads / 64; ++w) {
+            s += wave_acc[w];
+            b |= wave_bad_any[w];
+        }
+        agent_store(gaddr<double>(hdr->partials) + seg, s);
+        if (hdr->unscale) agent_store(gaddr<uint32_t>(hdr->nonfinite) + seg, b);
+        last_of_gradient = draw_ticket(tickets + t) == (uint32_t)(end - T.seg_start) - 1u ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!last_of_gradient) return;
+    if (threadIdx.x < 64) {
+        const double norm_sq = norm_tensor_sq(hdr, T.seg_start, end, dtype);
+        if (threadIdx.x == 0) {
+            agent_store(gaddr<double>(hdr->norm_sq) + t, norm_sq);
+            last_of_all = draw_ticket(tickets + count) == (uint32_t)count - 1u ? 1u : 0u;
+        }
+    }
+    __syncthreads();
+    if (last_of_all) norm_finish(hdr, wave_acc, wave_bad_any);
+}
+
+__global__ void __launch_bounds__(kNormThreads) norm_kernel(const NormHeader* hdr) { norm_body(hdr); }
+
+// The same with header and rows in the launch's arguments (few gradients: no staging copy before it).
+constexpr int kNormInlineBytes = 3840;
+struct __align__(16) NormInlineArgs {
+    unsigned char table[kNormInlineBytes];
+};
+__global__ void __launch_bounds__(kNormThreads) norm_kernel_inline(const NormInlineArgs a) {
+    norm_body((const NormHeader*)((const char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(NormInlineArgs, table)));
 }
 
 }  // namespace aw4

@@ -626,6 +626,7 @@ struct StagingSlot {
     const void* host_dev = nullptr;  // the device's address of `host`
     void* dev = nullptr;             // device copy the kernels read
     size_t cap = 0;
+    uint32_t* tickets = nullptr;     // the norm pass's workgroup counters, behind `dev`: zero outside its launches
     hipEvent_t done = nullptr;
     bool pending = false;
 };
@@ -927,7 +928,11 @@ int acquire_slot(DeviceState* ds, size_t bytes, StagingSlot** out) {
         void* mapped = nullptr;
         AW4_HIP_CHECK(hipHostGetDevicePointer(&mapped, slot.host, 0));
         slot.host_dev = mapped;
-        AW4_HIP_CHECK(hipMalloc(&slot.dev, cap));
+        // The counters: one per gradient and one more, of a pass that keeps 8 bytes per gradient in `dev`.
+        const std::vector<uint32_t> zero(cap / 8 + 1, 0u);
+        AW4_HIP_CHECK(hipMalloc(&slot.dev, cap + zero.size() * sizeof(uint32_t)));
+        slot.tickets = (uint32_t*)((char*)slot.dev + cap);
+        AW4_HIP_CHECK(hipMemcpy(slot.tickets, zero.data(), zero.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         slot.cap = cap;
     }
     // The event only tells the host that the launch which read the slot has finished; no data
@@ -1269,6 +1274,17 @@ int aw4_dequantize(const aw4_moment* m, int64_t numel, float* out, void* stream)
 
 namespace {
 
+// Segments of 2^18 gradient values for large models, shorter ones (to 2^13) while the launch would have
+// fewer than eight workgroups per CU: at 2^18 one 4096^2 gradient is 64 workgroups for 256 CUs, and
+// GPT-2-small's 124M values 585, an uneven two or three per CU.
+int norm_segment_shift(int64_t values) {
+    int shift = kNormShiftMin;
+    while (shift < kNormShiftMax && (values >> (shift + 1)) >= 2048) ++shift;
+    return shift;
+}
+
+int64_t norm_segments(int64_t numel, int shift) { return (numel + ((int64_t)1 << shift) - 1) >> shift; }
+
 // The norm pass and coefficient of aw4_clip_coefficient (inv_scale null) and
 // aw4_unscale_clip_coefficient.
 int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, const float* inv_scale,
@@ -1281,7 +1297,7 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
         (unscale && (!aligned((uint64_t)inv_scale, 4) || !aligned((uint64_t)found_out, 4))))
         return set_error(AW4_EALIGN, "%s: device floats not 4-byte aligned", what);
     int result_dtype = tensors[0].grad_dtype;
-    int64_t segments = 0;
+    int64_t values = 0;
     for (int i = 0; i < count; ++i) {
         const aw4_tensor& t = tensors[i];
         if (!t.grad || t.numel <= 0) return set_error(AW4_EINVAL, "tensor %d: null grad or numel %lld", i,
@@ -1291,14 +1307,18 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
         if ((t.flags & AW4_TENSOR_VEC_ALIGNED) && !aligned(t.grad, t.grad_dtype == AW4_F32 ? 16 : 8))
             return set_error(AW4_EALIGN, "tensor %d: VEC_ALIGNED but grad misaligned", i);
         if (t.grad_dtype != result_dtype) result_dtype = AW4_F32;  // torch.stack promotes mixed dtypes
-        segments += (t.numel + kNormSegment - 1) / kNormSegment;
+        values += t.numel;
     }
+    const int shift = norm_segment_shift(values);
+    int64_t segments = 0;
+    for (int i = 0; i < count; ++i) segments += norm_segments(tensors[i].numel, shift);
     if (segments > 0x7fffffff) return set_error(AW4_EINVAL, "%s: too many segments", what);
-    // staging: header, rows, segment starts (copied), then the partial sums, the per-gradient
-    // squared norms and (unscaling) the per-segment non-finite flags (device only)
-    const size_t table = (sizeof(NormHeader) + sizeof(aw4_tensor) * count + sizeof(int64_t) * (count + 1) + 255) &
-                         ~(size_t)255;
-    const size_t bytes = table + sizeof(double) * ((size_t)segments + (size_t)count) +
+    // header and rows (in the launch's arguments where they fit, else staged), then on the device the
+    // partial sums, the per-gradient squared norms and (unscaling) the per-segment non-finite flags
+    const size_t table = sizeof(NormHeader) + sizeof(NormRow) * (size_t)count;
+    const bool in_args = table <= (size_t)kNormInlineBytes;
+    const size_t scratch_at = in_args ? 0 : (table + 255) & ~(size_t)255;
+    const size_t bytes = scratch_at + sizeof(double) * ((size_t)segments + (size_t)count) +
                          (unscale ? sizeof(uint32_t) * (size_t)segments : 0);
 
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -1308,24 +1328,26 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     StagingSlot* slot = nullptr;
     rc = acquire_slot(ds, bytes, &slot);
     if (rc) return rc;
-    NormHeader* h = (NormHeader*)slot->host;
+    NormInlineArgs args;
+    NormHeader* h = (NormHeader*)(in_args ? (void*)args.table : slot->host);
     memset(h, 0, sizeof(*h));
-    aw4_tensor* rows = (aw4_tensor*)(h + 1);
-    int64_t* starts = (int64_t*)(rows + count);
+    NormRow* rows = (NormRow*)(h + 1);
     int64_t acc = 0;
     for (int i = 0; i < count; ++i) {
-        rows[i] = tensors[i];
-        starts[i] = acc;
-        acc += (tensors[i].numel + kNormSegment - 1) / kNormSegment;
+        const aw4_tensor& t = tensors[i];
+        rows[i] = NormRow{t.grad, t.numel, (int32_t)acc,
+                          t.grad_dtype | ((t.flags & AW4_TENSOR_VEC_ALIGNED) ? kNormVec : 0)};
+        acc += norm_segments(t.numel, shift);
     }
-    starts[count] = acc;
     h->count = count;
     h->result_dtype = result_dtype;
     h->max_norm = max_norm;
     h->unscale = unscale ? 1 : 0;
-    h->total_segments = segments;
-    h->partials = (uint64_t)slot->dev + table;
+    h->total_segments = (int32_t)segments;
+    h->segment_shift = shift;
+    h->partials = (uint64_t)slot->dev + scratch_at;
     h->norm_sq = h->partials + sizeof(double) * (uint64_t)segments;
+    h->tickets = (uint64_t)slot->tickets;
     h->norm_out = (uint64_t)norm_out;
     h->coef_out = (uint64_t)coef_out;
     if (unscale) {
@@ -1334,14 +1356,13 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
         h->found_out = (uint64_t)found_out;
     }
     hipStream_t s = (hipStream_t)stream;
-    rc = upload_slot(*slot, table, s);
-    if (rc) return rc;
-    const NormHeader* dh = (const NormHeader*)slot->dev;
-    hipLaunchKernelGGL(norm_partials_kernel, dim3((unsigned)segments), dim3(kNormThreads), 0, s, dh);
-    AW4_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(norm_tensor_kernel, dim3((unsigned)count), dim3(64), 0, s, dh);
-    AW4_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(norm_finish_kernel, dim3(1), dim3(kNormThreads), 0, s, dh);
+    if (in_args) {
+        hipLaunchKernelGGL(norm_kernel_inline, dim3((unsigned)segments), dim3(kNormThreads), 0, s, args);
+    } else {
+        rc = upload_slot(*slot, table, s);
+        if (rc) return rc;
+        hipLaunchKernelGGL(norm_kernel, dim3((unsigned)segments), dim3(kNormThreads), 0, s, (const NormHeader*)slot->dev);
+    }
     AW4_HIP_CHECK(hipGetLastError());
     AW4_HIP_CHECK(hipEventRecord(slot->done, s));
     slot->pending = true;

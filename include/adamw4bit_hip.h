@@ -250,8 +250,8 @@ int aw4_uniforms(uint64_t seed, uint64_t offset, int64_t n, float* out, void* st
  *   total  = sqrt(sum_t norm_t^2) rounded to R, the promotion of all gradient dtypes,
  *   coef   = min(RN(RN(1 / RN(total + 1e-6)) * max_norm), 1), each op rounded to R
  *            (clip_grad.py: max_norm / (total_norm + 1e-6) is reciprocal then multiply).
- * Sums of squares are taken in float64 in a fixed order (the result does not depend on
- * the launch shape).  Writes the fp32 values of total to norm_out[0] and of coef to
+ * Sums of squares are taken in float64 in an order fixed by the gradients' sizes (the result
+ * does not depend on how the launch runs).  Writes the fp32 values of total to norm_out[0] and of coef to
  * coef_out[0] (device addresses) without a host synchronisation.  Put coef in the second
  * float of the rows' grad_scale pair (AW4_TENSOR_GRAD_SCALE) of the next aw4_fused_step: the
  * step then reads the clipped gradients the in-place _foreach_mul_ would have written, and

@@ -124,3 +124,28 @@ def test_codec_sizes_match_oracle(mode, eden, blocks):
     levels = q.codebook_tensor(mode)
     assert torch.equal(H.bits(out[:values.numel()]), H.bits(levels[expect.long()] * expect_scales.repeat_interleave(128)))
     assert bool((out[values.numel():] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [[1], [3], [8191, 8193, 5], [4096 * 4096], [1 << 18] * 9 + [1000001],
+                                   [257 * (i % 7 + 1) for i in range(156)],   # the most rows launch arguments hold
+                                   [257 * (i % 7 + 1) for i in range(157)],   # one more: a staged table
+                                   [40_000_003, 11, 30_000_000]])
+def test_clip_norm_sizes(sizes, dtype):
+    """The norm pass over segments of 2^13 to 2^15 values, cut ones, many gradients and one; twice, since
+    its counters must be zero again.  The same gradients one value off their alignment, too."""
+    gen = torch.Generator(device=H.DEVICE).manual_seed(len(sizes))
+    for shift in (0, 1):
+        params = []
+        for n in sizes:
+            p = torch.nn.Parameter(torch.zeros(n, device=H.DEVICE, dtype=dtype))
+            p.grad = torch.randn(n + 4, generator=gen, device=H.DEVICE).to(dtype)[shift:shift + n]
+            params.append(p)
+        opt = aw.ZEEDENAdamW4Bit(params, optimized=True)
+        per = [p.grad.double().square().sum().sqrt().float().to(dtype) for p in params]
+        want = torch.stack([x.double() for x in per]).square().sum().sqrt().float().to(dtype)
+        for _ in range(6):  # every staging slot, and the first one again
+            norm = opt.clip_grad_norm_(1.0)
+            opt._grad_clip = None  # no step: drop the pending clip
+            torch.cuda.synchronize()
+            assert torch.equal(norm, want), (sizes, float(norm), float(want))
