@@ -66,12 +66,45 @@ struct __align__(16) LutEntry {
     float lv_hi;
 };
 
+// The specialised kernels' lookup table: bucket k of |x| <= 1 is the k-th step of the grid that
+// x + magic (one addition) rounds x to, magic = 1.5 * 2^m with an ulp of 2^(m - 23) = the bucket width, so
+// that the bucket is in the sum's low bits and its entry's address one shift and addition more: two
+// instructions, where the exponent and mantissa buckets of LutEntry, which hold any x, take five (three
+// for x >= 0).  Code or level count = base + (x >= thr), as there.  The width is the widest power of two
+// from 1/16 to 1/512 with at most one change per bucket (build_linear_lut).  With the value-space SR
+// entries below: GPT-2-small under ZE-EDEN with clipping 428 -> 414 us (128 -> 96 VGPRs, five waves per
+// SIMD), two Llama-3-8B layers under ZIP-SR bf16 848 -> 832 us, a bf16 set with an nf4_sr head of 525M
+// values 1,720 -> 1,652 us, one layer under the proxy lookahead 746 -> 733 us.
+struct __align__(8) LinEntry {
+    float thr;
+    uint32_t base;
+};
+constexpr int kLinSlots = 514;  // LDS entries: a signed codebook at 1/256, an unsigned one at 1/512
+
+struct LinTable {
+    float magic;
+    int32_t count;  // entries: 2 / width + 1 of a signed codebook (bucket of -1 first), 1 / width + 1 else
+    int32_t zero;   // the entry of x = 0
+    int32_t reserved;
+    LinEntry e[kLinSlots];
+};
+
 // Neighbouring levels of a searchsorted-left index (_compiled_quantization.py:30-38).
 struct __align__(16) PairEntry {
     float a;          // cb[lo]
     float b;          // cb[hi]
     float width_rcp;  // RN(1 / max(b - a, 1e-12))
     uint32_t lohi;    // lo | hi << 8
+};
+
+// Value-space stochastic rounding for each searchsorted index i >= 1: P(hi) * 2^24 = RN((x - a) / width),
+// width = RN(b - a) * 2^-24 (the scaling is exact, so the quotient is RN((x - a) / RN(b - a)) * 2^24).
+// Entry 0 (no level below x) gives a P above every draw, so that its code, idx - lower, is 0.
+struct __align__(16) SsrEntry {
+    float a;          // cb[lo]
+    float width;
+    float width_rcp;  // RN(1 / width)
+    float reserved;
 };
 
 // Per-block update-SR quantities for each searchsorted index i (update_sr_tables()), with
@@ -96,6 +129,7 @@ struct Tables {
     float codebook[AW4_NUM_CODEBOOKS][16];
     UsrPair usr[AW4_NUM_CODEBOOKS][kPairs];  // per searchsorted index (update-SR)
     PairEntry pairs[AW4_NUM_CODEBOOKS][kPairs];
+    SsrEntry ssr[AW4_NUM_CODEBOOKS][kPairs];  // per searchsorted index (value-space SR)
     float2 dec[AW4_NUM_CODEBOOKS][256];  // code byte -> (level of low nibble, level of high nibble)
     LutEntry lut[AW4_NUM_LUTS][AW4_LUT_ENTRIES];
 };
@@ -107,7 +141,22 @@ struct MomentTables {
     const float2* dec;
     const LutEntry* lut;
     const UsrPair* usr;
+    const SsrEntry* ssr;
+    // LinEntry table (specialised kernels): magic, and the LDS address of an entry less 8 * the bits of
+    // x + magic
+    float lin_magic;
+    uint32_t lin_base;
 };
+
+typedef const u32x2 __attribute__((address_space(3))) * LinLds;
+
+// The table entry of |x| <= 1 (kNonNeg: of |x|, so that it lies in an unsigned codebook's table whatever
+// x is).
+template <bool kNonNeg>
+__device__ __forceinline__ LinEntry lin_lookup(const MomentTables& L, float x) {
+    const u32x2 w = *(LinLds)(L.lin_base + (f2u((kNonNeg ? __builtin_fabsf(x) : x) + L.lin_magic) << 3));
+    return LinEntry{u2f(w.x), w.y};
+}
 
 // LDS scratch of one block's encode: update-SR tables of the block and the staging area
 // of its 64 code bytes (written a quarter at a time, stored to memory in one piece).
@@ -146,6 +195,25 @@ __device__ __forceinline__ int lut_bucket_unsigned(float x) { return lut_field(f
 __device__ __forceinline__ int lut_bucket_signed(float x) {
     const uint32_t u = f2u(x);
     return lut_field(u) - (AW4_LUT_EXP0 - 1) + (int)(u >> 31) * AW4_LUT_HALF;
+}
+
+// Off the fast path (blocks whose scale is not normal; IEEE division) x may be NaN: a LinEntry table takes
+// it as the top level 1, whose round-to-nearest code is the top one too, and its searchsorted index is
+// then set to 16, above every level.  The empty asm statements keep both in their uniform branch (hipcc
+// otherwise makes them selects that every value pays for).
+__device__ __forceinline__ void lin_arguments(bool wave_fast, float (&x)[4]) {
+    if (__builtin_expect(!wave_fast, 0)) {
+        asm volatile("");
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[t] = x[t] != x[t] ? 1.0f : fminf(fmaxf(x[t], -1.0f), 1.0f);
+    }
+}
+__device__ __forceinline__ void lin_nan_indexes(bool wave_fast, const float (&x)[4], int (&idx)[4]) {
+    if (__builtin_expect(!wave_fast, 0)) {
+        asm volatile("");
+#pragma unroll
+        for (int t = 0; t < 4; ++t) idx[t] = x[t] != x[t] ? 16 : idx[t];
+    }
 }
 
 // Decode the 4 values of one 16-bit code word: two LDS reads of level pairs.
@@ -331,7 +399,8 @@ struct BlockScales {
     float stored;
 };
 
-template <int SPEC, bool kNonNeg, class Values>
+// kLin: the moment's table is a LinEntry one (the specialised step kernels).
+template <int SPEC, bool kNonNeg, bool kLin = false, class Values>
 __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const MomentTables& L, int64_t blk0, int grp,
                                                     int j, bool active, const Values& vals, BlockScratch sc) {
     // max |m| over the lane's values, then over the block's 8 lanes on the bit patterns
@@ -377,16 +446,24 @@ __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const M
                 x[t] = v != v ? __builtin_nanf("") : v;
             }
         }
+        float xl[4] = {x[0], x[1], x[2], x[3]};  // what the lookup takes
+        if constexpr (kLin) lin_arguments(wave_fast, xl);
         uint32_t code[4];
         float lv[4];
         if constexpr (KIND == K_RTN) {
             // code = base + (x >= thr); the level for EDEN comes with the entry.
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const LutEntry e = L.lut[kNonNeg ? lut_bucket_unsigned(x[t]) : lut_bucket_signed(x[t])];
-                const bool up = x[t] >= e.thr;
-                code[t] = e.base + (up ? 1u : 0u);
-                lv[t] = up ? e.lv_hi : e.lv_lo;
+                if constexpr (kLin) {
+                    const LinEntry e = lin_lookup<kNonNeg>(L, xl[t]);
+                    code[t] = e.base + (xl[t] >= e.thr ? 1u : 0u);
+                    lv[t] = eden ? L.cb[code[t]] : 0.0f;
+                } else {
+                    const LutEntry e = L.lut[kNonNeg ? lut_bucket_unsigned(x[t]) : lut_bucket_signed(x[t])];
+                    const bool up = x[t] >= e.thr;
+                    code[t] = e.base + (up ? 1u : 0u);
+                    lv[t] = up ? e.lv_hi : e.lv_lo;
+                }
             }
         } else {
             float u[4];  // the uniforms times 2^24
@@ -397,10 +474,27 @@ __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const M
             int idx[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const LutEntry le = L.lut[kNonNeg ? lut_bucket_unsigned(x[t]) : lut_bucket_signed(x[t])];
-                idx[t] = (int)le.base + (x[t] >= le.thr ? 1 : 0);
+                if constexpr (kLin) {
+                    const LinEntry le = lin_lookup<kNonNeg>(L, xl[t]);
+                    idx[t] = (int)le.base + (xl[t] >= le.thr ? 1 : 0);
+                } else {
+                    const LutEntry le = L.lut[kNonNeg ? lut_bucket_unsigned(x[t]) : lut_bucket_signed(x[t])];
+                    idx[t] = (int)le.base + (x[t] >= le.thr ? 1 : 0);
+                }
             }
-            if constexpr (KIND == K_SSR) {
+            if constexpr (kLin) lin_nan_indexes(wave_fast, x, idx);
+            if (KIND == K_SSR && __builtin_expect(wave_fast, 1)) {
+                // P(hi) * 2^24 from the index's entry, without the guards and clamps, which change no
+                // code here: with |x| <= 1, the top level of every codebook, idx is at most 15; a level
+                // below x (idx >= 1) makes x > a, and x == b gives P = 1, above every draw; idx = 0 is
+                // entry 0's.  (Twelve vector instructions a value with them, six so.)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const SsrEntry se = L.ssr[idx[t]];
+                    const bool lower = !(u[t] < div_by_rcp(x[t] - se.a, se.width, se.width_rcp));
+                    code[t] = (uint32_t)(idx[t] - (lower ? 1 : 0));
+                }
+            } else if constexpr (KIND == K_SSR) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     // P(hi) = (x - a) / max(b - a, 1e-12), 0 where b == a (there lo == hi); guards
@@ -609,7 +703,8 @@ __device__ __forceinline__ void la_quick(const LaQuick& k, float z, float a, flo
 // Lookahead update-SR of this lane's 16 values z of block blk0 + grp (clamped at 0 first).
 // fresh: (1-beta2) * g^2 in float64 from the gradients g, or with AW4_MOMENT_FRESH_PROXY
 // fp32(w2f * z) (the v-proxy's (1 - beta2) * m2, fp32(1-beta2) = w2f).  Stores the codes
-// and scale (store), and/or returns each value's sample fp32(s * level) (sampled).
+// and scale (store), and/or returns each value's sample fp32(s * level) (sampled).  kLin as encode_block.
+template <bool kLin>
 __device__ __forceinline__ BlockScales encode_block_la(const aw4_moment& M, const MomentTables& L, int64_t blk0,
                                                        int grp, int j, bool active, const float (&z_in)[16],
                                                        const float (&g)[16], float w2f, bool store, float* sampled,
@@ -644,16 +739,38 @@ __device__ __forceinline__ BlockScales encode_block_la(const aw4_moment& M, cons
         float a[4], b[4];
         bool lower[4];
         uint64_t unsure = quick ? 0 : ~0ull;  // lanes (bits) with a value the quick form leaves open
+        float xq[4], xl[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const int i = 4 * q + t;
-            const float xq = __builtin_expect(wave_fast, 1) ? div_by_rcp(z[i], s, y) : z[i] / s;
-            const float x = clamp01_nan(xq);
-            const LutEntry le = L.lut[lut_bucket_unsigned(x)];
-            const bool up = x >= le.thr;
-            idx[t] = (int)le.base + (up ? 1 : 0);
-            b[t] = up ? le.lv_hi : le.lv_lo;   // cb[min(idx, 15)]
-            a[t] = L.cb[idx[t] > 0 ? idx[t] - 1 : 0];
+            xq[t] = __builtin_expect(wave_fast, 1) ? div_by_rcp(z[i], s, y) : z[i] / s;
+            xl[t] = xq[t];
+        }
+        if constexpr (kLin) {
+            // 0 <= z <= s: x is in [0, 1] as it is, except NaN off the fast path
+            lin_arguments(wave_fast, xl);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const LinEntry le = lin_lookup<true>(L, xl[t]);
+                idx[t] = (int)le.base + (xl[t] >= le.thr ? 1 : 0);
+            }
+            lin_nan_indexes(wave_fast, xq, idx);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int i = 4 * q + t;
+            if constexpr (kLin) {
+                const PairEntry pe = L.pairs[idx[t]];  // cb[max(idx - 1, 0)], cb[min(idx, 15)]
+                a[t] = pe.a;
+                b[t] = pe.b;
+            } else {
+                const float x = clamp01_nan(xq[t]);
+                const LutEntry le = L.lut[lut_bucket_unsigned(x)];
+                const bool up = x >= le.thr;
+                idx[t] = (int)le.base + (up ? 1 : 0);
+                b[t] = up ? le.lv_hi : le.lv_lo;   // cb[min(idx, 15)]
+                a[t] = L.cb[idx[t] > 0 ? idx[t] - 1 : 0];
+            }
             if (quick) {
                 const float fresh = proxy ? clamp_min_nan(w2f * z_in[i], 0.0f) : (wf * g[i]) * g[i];
                 bool sure;

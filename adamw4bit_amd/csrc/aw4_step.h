@@ -22,6 +22,8 @@ enum : int { D_F32 = AW4_F32, D_BF16 = AW4_BF16, D_F16 = AW4_F16, D_F64 = AW4_F6
 struct StepHeader {
     int32_t count;
     int32_t cb1, lut1, cb2, lut2;  // codebook / lookup table of each moment (specialised kernels)
+    float lin_magic[2];            // of each moment's LinTable, and the entry of x = 0
+    int32_t lin_zero[2];
     int32_t reserved;
     int64_t total_tiles;
     int64_t tiles_per_wave;
@@ -468,7 +470,7 @@ template <int MK, bool kNonNeg, class Values>
 __device__ __forceinline__ BlockScales encode_moment(const aw4_moment& M, const MomentTables& L, const TileLane& tl,
                                                      const Values& v, BlockScratch sc) {
     if constexpr (kind_of(MK) == K_ANY) return encode_block_any<kNonNeg>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
-    else return encode_block<MK, kNonNeg>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
+    else return encode_block<MK, kNonNeg, true>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
 }
 
 // Where the update puts the new second moments: registers, or this lane's slots of an LDS
@@ -850,8 +852,8 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
             const TileLane tl = tile_lane(T, local * kBlocksPerWave, lane);
             if (!loaded) load_tile(T, tl, in);
             codes_to_lanes(T, tl, in, ws);
-            const MomentTables L1 = lds_tables.moment(T.m1, 0);
-            const MomentTables L2 = lds_tables.moment(T.m2, 1);
+            const MomentTables L1 = lds_tables.moment(T.m1, 0, hdr);
+            const MomentTables L2 = lds_tables.moment(T.m2, 1, hdr);
             auto prefetch = [&]() {
                 loaded = false;
                 if (kPrefetch && more) {
@@ -889,6 +891,7 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
                     // lookahead update-SR: sample the pending state before the update (the
                     // generic instance, or the K_LA instance specialised on AW4_MOMENT_PENDING),
                     // or encode the new m2 after it (the code-storing proxies)
+                    constexpr bool kLin = kind_of(M2K) == K_LA;
                     constexpr bool kMaybePending = kind_of(M2K) == K_ANY || pending_spec(M2K);
                     float g[16];
                     tile_grads(T, in, g);
@@ -901,7 +904,7 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
                             float z[16];
 #pragma unroll
                             for (int i = 0; i < 16; ++i) z[i] = in.v2[i];
-                            encode_block_la(T.m2, L2, tl.blk0, tl.grp, tl.j, tl.active, z, g, w2f, false, prior,
+                            encode_block_la<kLin>(T.m2, L2, tl.blk0, tl.grp, tl.j, tl.active, z, g, w2f, false, prior,
                                             ws.block(tl.grp));
                         }
                     }
@@ -917,7 +920,7 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
                     }
                     if constexpr (!pending_spec(M2K)) {
                         if (!stored)
-                            encode_block_la(T.m2, L2, tl.blk0, tl.grp, tl.j, tl.active, m2v, g, w2f, true, nullptr,
+                            encode_block_la<kLin>(T.m2, L2, tl.blk0, tl.grp, tl.j, tl.active, m2v, g, w2f, true, nullptr,
                                             ws.block(tl.grp));
                     }
                   }

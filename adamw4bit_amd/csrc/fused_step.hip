@@ -54,7 +54,7 @@
 // hipGetSymbolAddress (device_state) and uses only that.  (Only the main object holds them: the
 // second compile of this file, AW4_SCHED_ILP_TU below, emits kernels and nothing else.)
 #ifndef AW4_SCHED_ILP_TU
-static __device__ __align__(256) uint8_t g_tables_mem[sizeof(aw4::Tables)];
+static __device__ __align__(256) uint8_t g_tables_mem[sizeof(aw4::Tables) + AW4_NUM_LUTS * sizeof(aw4::LinTable)];
 static __device__ __align__(256) uint8_t scratch[AW4_NOALLOC_TABLE_BYTES];
 #endif
 
@@ -92,19 +92,26 @@ __host__ __device__ inline int lut_id_of(int rounding, int codebook, int flags) 
 // LDS layouts
 // ---------------------------------------------------------------------------
 
+// The LinTable of every lookup-table id, behind the other tables.
+__host__ __device__ inline const LinTable* lin_tables(const Tables* g) { return (const LinTable*)(g + 1); }
+
 // Specialised kernels: the tables of the one codebook each moment uses.
-template <bool kUpd>
+template <bool kUpd, bool kSsr>
 struct LdsSlots {
     float cb[2][16];
     UsrPair usr[2][kPairs];
     PairEntry pairs[2][kPairs];
+    SsrEntry ssr[kSsr ? 2 : 1][kPairs];
     float2 dec[2][256];
-    LutEntry lut[2][AW4_LUT_ENTRIES];
+    LinEntry lin[2][kLinSlots];
     WaveScratch scratch[kWavesPerGroup];
     f32x4 m2_stage[kUpd ? kWavesPerGroup * 4 * 64 : 1];  // second moments of a tile (update-SR kernels)
 
-    __device__ MomentTables moment(const aw4_moment&, int which) const {
-        return MomentTables{cb[which], pairs[which], dec[which], lut[which], usr[which]};
+    __device__ __forceinline__ MomentTables moment(const aw4_moment&, int which, const StepHeader* h) const {
+        const float magic = h->lin_magic[which];
+        const uint32_t at = (uint32_t)(uintptr_t)(LinLds)(&lin[which][0]);
+        return MomentTables{cb[which], pairs[which], dec[which], nullptr, usr[which], ssr[kSsr ? which : 0], magic,
+                            at + ((uint32_t)h->lin_zero[which] << 3) - (f2u(magic) << 3)};
     }
     __device__ f32x4* wave_m2_stage(int wslot) { return kUpd ? &m2_stage[wslot * 4 * 64] : nullptr; }
     __device__ void load(const Tables* g, const StepHeader* h) {
@@ -114,8 +121,12 @@ struct LdsSlots {
             for (int i = threadIdx.x; i < 16; i += kThreads) cb[w][i] = g->codebook[cbs[w]][i];
             for (int i = threadIdx.x; i < kPairs; i += kThreads) usr[w][i] = g->usr[cbs[w]][i];
             for (int i = threadIdx.x; i < kPairs; i += kThreads) pairs[w][i] = g->pairs[cbs[w]][i];
+            if (kSsr)
+                for (int i = threadIdx.x; i < kPairs; i += kThreads) ssr[w][i] = g->ssr[cbs[w]][i];
             for (int i = threadIdx.x; i < 256; i += kThreads) dec[w][i] = g->dec[cbs[w]][i];
-            for (int i = threadIdx.x; i < AW4_LUT_ENTRIES; i += kThreads) lut[w][i] = g->lut[luts[w]][i];
+            const LinTable& lt = lin_tables(g)[luts[w]];
+            const int n = lt.count;
+            for (int i = threadIdx.x; i < n; i += kThreads) lin[w][i] = lt.e[i];
         }
         __syncthreads();
     }
@@ -126,11 +137,11 @@ struct LdsAll {
     Tables t;
     WaveScratch scratch[kWavesPerGroup];
 
-    __device__ __forceinline__ MomentTables moment(const aw4_moment& m, int) const {
+    __device__ __forceinline__ MomentTables moment(const aw4_moment& m, int, const StepHeader*) const {
         const int cbid = m.rounding == AW4_ROUND_FP32 ? 0 : m.codebook;
         return MomentTables{t.codebook[cbid], t.pairs[cbid], t.dec[cbid],
                             t.lut[m.rounding == AW4_ROUND_FP32 ? 0 : lut_id_of(m.rounding, cbid, m.flags)],
-                            t.usr[cbid]};
+                            t.usr[cbid], t.ssr[cbid], 0.0f, 0u};
     }
     __device__ f32x4* wave_m2_stage(int) { return nullptr; }
     __device__ void load(const Tables* g, const StepHeader*) {
@@ -145,8 +156,9 @@ template <int M1K, int M2K, int D>
 struct KernelTraits {
     static constexpr int K1 = kind_of(M1K), K2 = kind_of(M2K);
     static constexpr bool kGeneric = K1 == K_ANY || K2 == K_ANY || D == D_ANY;
+    static constexpr bool kSsr = K1 == K_SSR || K2 == K_SSR;
     static constexpr bool kUpd = K1 == K_USR || K2 == K_USR || K1 == K_ANY || K2 == K_ANY;
-    using Lds = typename std::conditional<kGeneric, LdsAll, LdsSlots<kUpd>>::type;
+    using Lds = typename std::conditional<kGeneric, LdsAll, LdsSlots<kUpd, kSsr>>::type;
 };
 
 template <int M1K, int M2K, int D>
@@ -362,6 +374,7 @@ struct LdsEncode {
     float cb[16];
     UsrPair usr[kPairs];
     PairEntry pairs[kPairs];
+    SsrEntry ssr[kPairs];
     LutEntry lut[AW4_LUT_ENTRIES];
     WaveScratch scratch[kWavesPerGroup];
 
@@ -370,6 +383,7 @@ struct LdsEncode {
         if (threadIdx.x < kPairs) {
             usr[threadIdx.x] = g->usr[codebook][threadIdx.x];
             pairs[threadIdx.x] = g->pairs[codebook][threadIdx.x];
+            ssr[threadIdx.x] = g->ssr[codebook][threadIdx.x];
         }
         if (threadIdx.x < AW4_LUT_ENTRIES) lut[threadIdx.x] = g->lut[lut_id][threadIdx.x];
         __syncthreads();
@@ -403,7 +417,7 @@ __global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restr
     float next[16];
     if (tile < tiles) load(tile, next);
     lds.load(tables, M.codebook, lut_id_of(M.rounding, M.codebook, M.flags));
-    const MomentTables L{lds.cb, lds.pairs, nullptr, lds.lut, lds.usr};
+    const MomentTables L{lds.cb, lds.pairs, nullptr, lds.lut, lds.usr, lds.ssr, 0.0f, 0u};
     while (tile < tiles) {
         float m[16];
 #pragma unroll
@@ -521,6 +535,7 @@ int rtn_code(const float* cb, float x, bool floor_zero) {
 
 struct HostTables {
     Tables t;
+    LinTable lin[AW4_NUM_LUTS];  // behind `t`, as in device memory
     bool ok = false;
     std::string error;
 };
@@ -577,6 +592,59 @@ bool build_lut(LutEntry* out, F f, const float* cb, std::string& err) {
     return true;
 }
 
+// The LinTable of f, monotone non-decreasing, over [0, 1] or (is_signed) [-1, 1]: the widest buckets that
+// hold at most one change of f each.
+template <class F>
+bool build_linear_lut(LinTable& out, F f, bool is_signed, std::string& err) {
+    // floats of the range in order, and back
+    auto value = [](int32_t k) { return k < 0 ? -host_f((uint32_t)-k) : host_f((uint32_t)k); };
+    const int32_t one = 0x3f800000;
+    for (int inv = 16; inv <= 512; inv *= 2) {
+        const int count = is_signed ? 2 * inv + 1 : inv + 1;
+        if (count > kLinSlots) break;
+        memset(&out, 0, sizeof(out));
+        out.magic = 1.5f * (float)(1 << 23) / (float)inv;
+        out.count = count;
+        out.zero = is_signed ? inv : 0;
+        auto bucket = [&](int32_t k) {
+            const volatile float sum = value(k) + out.magic;  // rounded to fp32, as the kernel's addition
+            const float s = sum;
+            uint32_t a, b;
+            memcpy(&a, &s, 4);
+            memcpy(&b, &out.magic, 4);
+            return (int)(a - b) + out.zero;
+        };
+        // first float of the range at or above bucket b
+        auto first = [&](int b) {
+            int32_t lo = is_signed ? -one : 0, hi = one + 1;
+            while (lo < hi) {
+                const int32_t mid = lo + (hi - lo) / 2;
+                if (bucket(mid) >= b) hi = mid; else lo = mid + 1;
+            }
+            return lo;
+        };
+        bool ok = bucket(is_signed ? -one : 0) == 0 && bucket(one) == count - 1;
+        for (int b = 0; b < count && ok; ++b) {
+            const int32_t lo = first(b), hi = first(b + 1) - 1;
+            const int base = f(value(lo)), top = f(value(hi));
+            out.e[b].base = (uint32_t)base;
+            out.e[b].thr = host_f(0x7fc00000u);  // never reached
+            if (top == base + 1) {
+                int32_t bad = lo, good = hi;
+                while (good - bad > 1) {
+                    const int32_t mid = bad + (good - bad) / 2;
+                    if (f(value(mid)) == base + 1) good = mid; else bad = mid;
+                }
+                out.e[b].thr = value(good);
+            }
+            ok = lo <= hi && top <= base + 1;
+        }
+        if (ok) return true;
+    }
+    err = "no linear lookup table holds one code change per bucket";
+    return false;
+}
+
 const HostTables& host_tables() {
     static HostTables h;
     static std::once_flag once;
@@ -603,6 +671,16 @@ const HostTables& host_tables() {
                 const float w = p.b - p.a;
                 p.width_rcp = 1.0f / (w < 1e-12f ? 1e-12f : w);
                 p.lohi = (uint32_t)lo | ((uint32_t)hi << 8);
+                // (the 1e-12 floor of the width binds only where lo == hi: index 0, and 16, which no x <= 1 has)
+                SsrEntry& e = t.ssr[c][i];
+                if (i > 0) {
+                    e.a = p.a;
+                    e.width = ldexpf(w < 1e-12f ? 1e-12f : w, -24);
+                } else {
+                    e.a = -8.0f;
+                    e.width = 0x1p-24f;
+                }
+                e.width_rcp = 1.0f / e.width;
             }
             for (int b = 0; b < 256; ++b) t.dec[c][b] = make_float2(t.codebook[c][b & 15], t.codebook[c][b >> 4]);
         }
@@ -614,7 +692,14 @@ const HostTables& host_tables() {
         }
         if (ok) {
             const float* cb = t.codebook[AW4_CB_DYN4];
-            ok = build_lut(t.lut[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, cb, h.error);
+            ok = build_lut(t.lut[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, cb, h.error) &&
+                 build_linear_lut(h.lin[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, false, h.error);
+        }
+        for (int c = 0; c < AW4_NUM_CODEBOOKS && ok; ++c) {
+            const float* cb = t.codebook[c];
+            const bool is_signed = cb[0] < 0.0f;
+            ok = build_linear_lut(h.lin[kLutRtn[c]], [cb](float x) { return rtn_code(cb, x, false); }, is_signed, h.error) &&
+                 build_linear_lut(h.lin[kLutLevels[c]], [cb](float x) { return count_less(cb, x); }, is_signed, h.error);
         }
         h.ok = ok;
     });
@@ -665,7 +750,8 @@ int device_state(DeviceState** out) {
         void* stage = nullptr;
         AW4_HIP_CHECK(hipGetSymbolAddress(&tables, HIP_SYMBOL(g_tables_mem)));
         AW4_HIP_CHECK(hipGetSymbolAddress(&stage, HIP_SYMBOL(scratch)));
-        AW4_HIP_CHECK(hipMemcpy(tables, &ht.t, sizeof(Tables), hipMemcpyHostToDevice));
+        static_assert(offsetof(HostTables, lin) == sizeof(Tables), "one copy of both");
+        AW4_HIP_CHECK(hipMemcpy(tables, &ht.t, sizeof(Tables) + sizeof(ht.lin), hipMemcpyHostToDevice));
         ds.scratch = (uint8_t*)stage;
         ds.tables = (Tables*)tables;
     }
@@ -852,7 +938,10 @@ std::vector<LaunchGroup> plan_launches(const aw4_tensor* ts, int32_t count) {
         // flag at run time.
         int v = kGenericVariant;
         const bool vec16 = aligned(t.param, 16);
-        if (t.param_dtype == t.grad_dtype && (t.flags & AW4_TENSOR_VEC_ALIGNED))
+        // ... and their lookup tables hold [-1, 1] for signed codebooks only: a first moment on an
+        // unsigned one (no scheme has it) runs the generic kernel.
+        const bool m1_signed = t.m1.rounding == AW4_ROUND_FP32 || t.m1.codebook == AW4_CB_NF4 || t.m1.codebook == AW4_CB_SDYN4;
+        if (t.param_dtype == t.grad_dtype && (t.flags & AW4_TENSOR_VEC_ALIGNED) && m1_signed)
             for (int k = 0; k < kNumSpecialised; ++k)
                 if (kVariants[k].dtype == t.param_dtype && kVariants[k].m1 == s1 && kVariants[k].m2 == s2 &&
                     (vec16 || !lds_tile_io(kVariants[k].m1, kVariants[k].m2, kVariants[k].dtype))) {
@@ -1042,6 +1131,12 @@ int fill_step_tables(const aw4_tensor* tensors, StepLaunch& sl, int num_cus, voi
             return set_error(AW4_EINVAL, "aw4_fused_step: %lld tiles exceed one launch", (long long)acc);
         h->count = n;
         h->cb1 = lg.cb1; h->lut1 = lg.lut1; h->cb2 = lg.cb2; h->lut2 = lg.lut2;
+        for (int w = 0; w < 2; ++w) {
+            const int lut = w == 0 ? lg.lut1 : lg.lut2;
+            if (lut < 0) continue;
+            h->lin_magic[w] = host_tables().lin[lut].magic;
+            h->lin_zero[w] = host_tables().lin[lut].zero;
+        }
         h->total_tiles = acc;
         h->tiles_per_wave = tiles_per_wave;
     }
