@@ -399,8 +399,79 @@ struct BlockScales {
     float stored;
 };
 
-// kLin: the moment's table is a LinEntry one (the specialised step kernels).
-template <int SPEC, bool kNonNeg, bool kLin = false, class Values>
+// The common case of a block encode, without a branch: a wave whose blocks all have normal scales and whose
+// draws are the generator's.  Returns whether every value's code is settled; if not (update-SR, a value
+// inside its band: one wave tile in fifty on heavy-tailed second moments) the caller encodes the tile's
+// blocks again by the general rule, which overwrites the staged codes and the sums.  As one stretch of
+// code its four quarters' table lookups, random numbers and roots overlap; with the tests for the general
+// rule between them (three branches a quarter) they ran one after the other: two Llama-3-8B layers under
+// ZIP-SR bf16 832 -> 822 us, the bf16 set with an nf4_sr head 1,652 -> 1,637 us, embedding and a layer in
+// fp32 1,870 -> 1,842 us (start's code on that box).  Kernels with a round-to-nearest second moment keep
+// the loop below, which has one branch a quarter for them: as one stretch ZE-EDEN fp32 needed 107 VGPRs
+// instead of 96 and lost its fifth wave (GPT-2-small with clipping 414 -> 423 us).
+template <int KIND, bool kNonNeg, class Values>
+__device__ __forceinline__ bool encode_quick(const aw4_moment& M, const MomentTables& L, int64_t blk0, int grp, int j,
+                                             const Values& vals, float s, float y, const UsrBlock& ub, bool eden,
+                                             bool floor0, float (&acc_xx)[4], float (&acc_xl)[4], BlockScratch sc) {
+    uint64_t unsure = 0;  // lanes (bits) with a value the quick test leaves open
+    uint32_t rw[12];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float x[4];
+        uint32_t code[4];
+        vals.quarter(q, x);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            x[t] = div_by_rcp(x[t], s, y);
+            const LinEntry e = lin_lookup<kNonNeg>(L, x[t]);
+            code[t] = e.base + (x[t] >= e.thr ? 1u : 0u);  // the code, or the number of levels below x
+        }
+        if constexpr (KIND != K_RTN) {
+            float u[4];
+            if (q < 3) philox_tile_call(M.rng_seed, (M.rng_offset >> 7) + (uint64_t)blk0, grp, j, q, &rw[4 * q]);
+            lane_fields4(&rw[3 * q], u);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                bool lower;
+                if constexpr (KIND == K_SSR) {
+                    // P(hi) * 2^24 from the index's entry.  The guards and clamps of the general rule change no
+                    // code here: with |x| <= 1, the top level of every codebook, the index is at most 15; a
+                    // level below x (index >= 1) makes x > a, and x == b gives P = 1, above every draw; index
+                    // 0 has entry 0.
+                    const SsrEntry se = L.ssr[code[t]];
+                    lower = !(u[t] < div_by_rcp(x[t] - se.a, se.width, se.width_rcp));
+                } else {
+                    // Where the quick test is sure: code = idx - lower, without guards or clamps.  The block is
+                    // certain, so every interval is valid.  No level below x (idx = 0): Q is NaN and lower
+                    // false, code 0.  x at its upper level b (where both forms of the rule pick hi):
+                    // Q = (sqrt(b) - w) - u * g * E(b) with w within an ulp of sqrt(b), so a sure Q is negative
+                    // and lower false.  idx <= 15, as x <= 1.
+                    bool sure;
+                    lower = usr_quick(sc.upd[code[t]], ub, M.sr_eps, x[t], u[t], sure) > 0.0f;
+                    unsure |= __builtin_amdgcn_ballot_w64(!sure);
+                }
+                code[t] -= lower ? 1u : 0u;
+            }
+        }
+        if (floor0 && KIND != K_RTN) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) code[t] = max(code[t], 1u);
+        }
+        if (eden) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                acc_xx[t] = acc_xx[t] + x[t] * x[t];
+                acc_xl[t] = acc_xl[t] + x[t] * L.cb[code[t]];
+            }
+        }
+        sc.stage[8 * q + j] = (uint16_t)(code[0] | (code[1] << 4) | (code[2] << 8) | (code[3] << 12));
+    }
+    return unsure == 0;
+}
+
+// kLin: the moment's table is a LinEntry one (the specialised step kernels); kQuick: encode_quick is tried
+// first.
+template <int SPEC, bool kNonNeg, bool kLin = false, bool kQuick = false, class Values>
 __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const MomentTables& L, int64_t blk0, int grp,
                                                     int j, bool active, const Values& vals, BlockScratch sc) {
     // max |m| over the lane's values, then over the block's 8 lanes on the bit patterns
@@ -427,8 +498,18 @@ __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const M
     wave_lds_sync();  // the stage's previous contents have been read
 
     float acc_xx[4] = {0.0f, 0.0f, 0.0f, 0.0f}, acc_xl[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    bool settled = false;
+    if constexpr (kQuick) {
+        if (__builtin_expect(wave_fast & ((M.flags & AW4_MOMENT_EXT_DRAWS) == 0), 1))
+            settled = encode_quick<KIND, kNonNeg>(M, L, blk0, grp, j, vals, s, y, ub, eden, floor0, acc_xx, acc_xl, sc);
+        if (__builtin_expect(!settled, 0)) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc_xx[t] = acc_xl[t] = 0.0f;
+        }
+    }
     uint32_t rw[12];  // Philox words of this lane's position group (stochastic kinds)
     bool level_preconds = false;  // the block's table of level preconditioners is built (update-SR)
+    if (__builtin_expect(!settled, !kQuick))
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         float x[4], mq[4];
@@ -483,18 +564,7 @@ __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const M
                 }
             }
             if constexpr (kLin) lin_nan_indexes(wave_fast, x, idx);
-            if (KIND == K_SSR && __builtin_expect(wave_fast, 1)) {
-                // P(hi) * 2^24 from the index's entry, without the guards and clamps, which change no
-                // code here: with |x| <= 1, the top level of every codebook, idx is at most 15; a level
-                // below x (idx >= 1) makes x > a, and x == b gives P = 1, above every draw; idx = 0 is
-                // entry 0's.  (Twelve vector instructions a value with them, six so.)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const SsrEntry se = L.ssr[idx[t]];
-                    const bool lower = !(u[t] < div_by_rcp(x[t] - se.a, se.width, se.width_rcp));
-                    code[t] = (uint32_t)(idx[t] - (lower ? 1 : 0));
-                }
-            } else if constexpr (KIND == K_SSR) {
+            if constexpr (KIND == K_SSR) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     // P(hi) = (x - a) / max(b - a, 1e-12), 0 where b == a (there lo == hi); guards

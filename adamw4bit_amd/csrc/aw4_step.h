@@ -466,11 +466,11 @@ __device__ __forceinline__ void params_to_memory(const aw4_tensor& T, const Tile
     wave_lds_sync();  // the pieces are read before the encodes write the scratch
 }
 
-template <int MK, bool kNonNeg, class Values>
+template <int MK, bool kNonNeg, bool kQuick, class Values>
 __device__ __forceinline__ BlockScales encode_moment(const aw4_moment& M, const MomentTables& L, const TileLane& tl,
                                                      const Values& v, BlockScratch sc) {
     if constexpr (kind_of(MK) == K_ANY) return encode_block_any<kNonNeg>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
-    else return encode_block<MK, kNonNeg, true>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
+    else return encode_block<MK, kNonNeg, true, kQuick>(M, L, tl.blk0, tl.grp, tl.j, tl.active, v, sc);
 }
 
 // Where the update puts the new second moments: registers, or this lane's slots of an LDS
@@ -676,11 +676,11 @@ __device__ __forceinline__ void sampled_read_update(const aw4_tensor& T, const T
 }
 
 // Encode (or store, for an fp32-state moment) one moment of a tile.
-template <int MK, bool kNonNeg, class Values>
+template <int MK, bool kNonNeg, bool kQuick = false, class Values>
 __device__ __forceinline__ BlockScales finish_moment(const aw4_moment& M, const MomentTables& L, const TileLane& tl,
                                                      const Values& v, WaveScratch& ws) {
     if (moment_quantized<MK>(M)) {
-        if constexpr (kind_of(MK) != K_FP32) return encode_moment<MK, kNonNeg>(M, L, tl, v, ws.block(tl.grp));
+        if constexpr (kind_of(MK) != K_FP32) return encode_moment<MK, kNonNeg, kQuick>(M, L, tl, v, ws.block(tl.grp));
     } else if (tl.active) {
         const gptr<float> vals_tile = gaddr<float>(M.values) + tl.blk0 * kBlock;
 #pragma unroll
@@ -929,9 +929,9 @@ __device__ __forceinline__ void run_tiles(const StepHeader* hdr, const LdsT& lds
                 M2Staged m2{m2_stage + lane, 0.0f};
                 update_tile_any(T, tl, in, L1, L2, m1, m2, nullptr, nullptr, ws.code_words());
                 params_to_memory<M1K, M2K, D>(T, tl, ws);
-                finish_moment<M1K, false>(T.m1, L1, tl, RegValues{m1}, ws);
+                finish_moment<M1K, false, true>(T.m1, L1, tl, RegValues{m1}, ws);
                 prefetch();
-                finish_moment<M2K, true>(T.m2, L2, tl, m2.values(), ws);
+                finish_moment<M2K, true, true>(T.m2, L2, tl, m2.values(), ws);
             } else {
                 float m2v[16];
                 M2Regs m2{m2v};

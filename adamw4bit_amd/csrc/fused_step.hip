@@ -248,14 +248,13 @@ values_kernel_inline(const InlineArgs a) {
 
 }  // namespace
 
-// The four-wave update-SR kernels (ZIP-SR's fp32 and bf16 steps, the bf16 nf4_sr head and
-// EDEN-m2 ablation) come from a second compile of this file, with AW4_SCHED_ILP_TU defined and
-// LLVM's max-ilp machine scheduler (-mllvm -amdgpu-sched-strategy=max-ilp); that object holds
-// nothing else.  Bound by their instruction issue, they ran 1.2-1.5% faster under it (ZIP-SR on
-// the Llama-3-8B fp32 set 19.40-19.55 against 19.77-19.85 ms, the bf16 set 16.28-16.49 against
-// 16.49-16.72 ms per step; alternating processes on one box, five each), while ZE-EDEN spills
-// under it and ran 4% slower, so every other kernel keeps the default scheduler.  The main
-// object declares them and launches them through the variant table.
+// The bf16 update-SR kernels (ZIP-SR and its nf4_sr head) come from a second compile of this file, with
+// AW4_SCHED_ILP_TU defined and LLVM's max-ilp machine scheduler (-mllvm -amdgpu-sched-strategy=max-ilp);
+// that object holds nothing else.  Bound by their instruction issue, the bf16 kernels ran 1.2-1.5% faster
+// under it, while ZE-EDEN spilled (4% slower).  Since the update-SR encode is one stretch of code
+// (encode_quick), the fp32 one and the EDEN-m2 ablation spill under it too (37 and 4 registers) and keep
+// the default scheduler.  The main object declares these kernels and launches them through the variant
+// table.
 namespace aw4_ilp {
 template <int M1K, int M2K, int D>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
@@ -295,12 +294,9 @@ constexpr int kAnyResearch = mspec(K_ANY, AW4_MOMENT_SAMPLED_READ);
 #ifdef AW4_SCHED_ILP_TU
 }  // namespace
 
-template __global__ void aw4_ilp::step_kernel_4w<kRtn, kUsrGuarded, D_F32>(const aw4::StepHeader*, const aw4::Tables*);
 template __global__ void aw4_ilp::step_kernel_4w<kRtn, kUsrGuarded, D_BF16>(const aw4::StepHeader*, const aw4::Tables*);
 template __global__ void aw4_ilp::step_kernel_4w<kSsrGuarded, kUsrGuarded, D_BF16>(const aw4::StepHeader*,
                                                                                    const aw4::Tables*);
-template __global__ void aw4_ilp::step_kernel_4w<kRtn, kUsrGuardedEden, D_BF16>(const aw4::StepHeader*,
-                                                                                const aw4::Tables*);
 #else
 
 struct KernelVariant {
@@ -330,11 +326,11 @@ struct KernelVariant {
 // Plain round-to-nearest pairs likewise: the GPT-2-small fp32 set 545 -> 312 us (5.6 TB/s), a 4.3 GB
 // bf16 set 3,590 -> 2,245 us.
 const KernelVariant kVariants[] = {
-    AW4_VARIANT_I4W(kRtn, kRtnEden, D_F32),       AW4_VARIANT_ILP_I4W(kRtn, kUsrGuarded, D_F32),
+    AW4_VARIANT_I4W(kRtn, kRtnEden, D_F32),       AW4_VARIANT_I4W(kRtn, kUsrGuarded, D_F32),
     AW4_VARIANT_I4W(kRtn, kRtnEden, D_BF16),      AW4_VARIANT_ILP_I4W(kRtn, kUsrGuarded, D_BF16),
     AW4_VARIANT(kSsrGuarded, kUsrGuarded, D_F32), AW4_VARIANT_ILP(kSsrGuarded, kUsrGuarded, D_BF16),
     AW4_VARIANT(kRtn, kFp32, D_F32),              AW4_VARIANT(kRtn, kFp32, D_BF16),
-    AW4_VARIANT(kRtn, kUsrGuardedEden, D_F32),    AW4_VARIANT_ILP(kRtn, kUsrGuardedEden, D_BF16),
+    AW4_VARIANT(kRtn, kUsrGuardedEden, D_F32),    AW4_VARIANT_4W(kRtn, kUsrGuardedEden, D_BF16),
     AW4_VARIANT_4W(kRtn, kRtnEden, D_F16),        AW4_VARIANT_4W(kRtn, kUsrGuarded, D_F16),
     AW4_VARIANT_4W(kSsrGuarded, kUsrGuarded, D_F16),
     AW4_VARIANT(kRtn, kFp32, D_F16),              AW4_VARIANT_4W(kRtn, kUsrGuardedEden, D_F16),
