@@ -149,3 +149,14 @@ def test_clip_norm_sizes(sizes, dtype):
             opt._grad_clip = None  # no step: drop the pending clip
             torch.cuda.synchronize()
             assert torch.equal(norm, want), (sizes, float(norm), float(want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m2", ["dyn4_proxy_la_upd_sr", "dyn4_vproxy_la_upd_sr", "dyn4_upd_sr"])
+def test_16bit_research_kernels_match_oracle(m2, dtype):
+    """16-bit parameters under the code-storing lookahead and the read-back second moments."""
+    log(f"{dtype} nf4 / {m2} x 3 steps")
+    make = lambda ps: aw.QuantizedAdamW(ps, lr=1e-3, weight_decay=0.1, m1_quant_scheme="nf4", m2_quant_scheme=m2,  # noqa: E731
+                                        quant_rng_seed=3, optimized=True)
+    out = run_pair(make, SHAPES, dtype, 3, seed=3, zero_block_frac=0.02, grad_fn=fp16_safe)
+    compare_pair(*out, f"{dtype} nf4/{m2}", steps=3)
