@@ -130,13 +130,18 @@ def rows_of(table: np.ndarray) -> Rows:
     return rows
 
 
-def fused_step(table: np.ndarray, stream: int) -> None:
-    """Launch one fused step over the rows of ``table`` (dtype :data:`TENSOR`)."""
+def _table_ptr(table: np.ndarray) -> int:
+    """The host address of a table's rows (dtype :data:`TENSOR`)."""
     ptr = table.ptr if type(table) is Rows else None
     if ptr is None:
         assert table.dtype == TENSOR and table.flags.c_contiguous
         ptr = table.ctypes.data
-    check(library().aw4_fused_step(ptr, len(table), stream), "aw4_fused_step")
+    return ptr
+
+
+def fused_step(table: np.ndarray, stream: int) -> None:
+    """Launch one fused step over the rows of ``table`` (dtype :data:`TENSOR`)."""
+    check(library().aw4_fused_step(_table_ptr(table), len(table), stream), "aw4_fused_step")
 
 
 def fused_step_noalloc(table: np.ndarray, stream: int) -> None:
@@ -159,8 +164,7 @@ def dequantize(moment: np.ndarray, numel: int, out_ptr: int, stream: int) -> Non
 def clip_coefficient(table: np.ndarray, max_norm: float, norm_ptr: int, coef_ptr: int, stream: int) -> None:
     """Global gradient norm of the rows of ``table`` and the clipping coefficient, written to
     the device floats at ``norm_ptr`` and ``coef_ptr``."""
-    assert table.dtype == TENSOR and table.flags.c_contiguous
-    check(library().aw4_clip_coefficient(table.ctypes.data, len(table), max_norm, norm_ptr, coef_ptr, stream),
+    check(library().aw4_clip_coefficient(_table_ptr(table), len(table), max_norm, norm_ptr, coef_ptr, stream),
           "aw4_clip_coefficient")
 
 
@@ -169,8 +173,7 @@ def unscale_clip_coefficient(table: np.ndarray, inv_scale_ptr: int, max_norm: fl
     """``clip_coefficient`` over gradients scaled by a loss scale: each value is unscaled by the
     device float at ``inv_scale_ptr`` as it is read, and ``found_inf_ptr`` receives 1.0 if any
     scaled value is not finite."""
-    assert table.dtype == TENSOR and table.flags.c_contiguous
-    check(library().aw4_unscale_clip_coefficient(table.ctypes.data, len(table), inv_scale_ptr, max_norm, norm_ptr,
+    check(library().aw4_unscale_clip_coefficient(_table_ptr(table), len(table), inv_scale_ptr, max_norm, norm_ptr,
                                                  coef_ptr, found_inf_ptr, stream), "aw4_unscale_clip_coefficient")
 
 

@@ -31,6 +31,7 @@ from __future__ import annotations
 
 import array
 import bisect
+import contextlib
 import functools
 import itertools
 import math
@@ -268,6 +269,9 @@ class _StepConstants:
                                         dtype=np.uint32)
         return self._words
 
+    def words_bytes(self) -> bytes:
+        return self.words().tobytes()
+
     def m2_sr_values(self) -> tuple:
         """fp32 update-SR storage bias max(c, 1e-12), its correctly rounded reciprocal, and eps."""
         return self._m2_vals
@@ -302,6 +306,11 @@ try:
 except ImportError:  # pragma: no cover - other torch builds
     def _raw_stream(index: int) -> int:
         return torch.cuda.current_stream(index).cuda_stream
+
+
+def _current_device(index: int):
+    """``torch.cuda.device(index)``, or nothing where it is current already."""
+    return contextlib.nullcontext() if torch.cuda.current_device() == index else torch.cuda.device(index)
 
 
 def _launch(params: List[torch.Tensor], written: List[torch.Tensor], read: List[torch.Tensor],
@@ -506,6 +515,7 @@ class QuantizedAdamW(Optimizer):
         # on-device Philox draws of a stochastic write (bit-exact comparisons with fed draws).
         self._draw_provider = None
         self._launch_plan: Optional[_LaunchPlan] = None
+        self._clip_plan: Optional[_ClipPlan] = None
         self._pending_finish = None  # commit / undo of the step being launched
         self._inconsistent: Optional[str] = None  # why step() refuses to run (a partly enqueued step)
         # Gradient clipping computed by clip_grad_norm_ and applied by the next step:
@@ -795,17 +805,16 @@ class QuantizedAdamW(Optimizer):
             if torch.compiler.is_compiling():
                 _ops.unscale_clip_coefficient_(grads, out, table, max_norm)
             else:
-                with torch.cuda.device(out.device):
+                with _current_device(out.device.index):
                     p = out.data_ptr()
-                    _lib.unscale_clip_coefficient(table.numpy().view(_lib.TENSOR), p + 8, max_norm, p, p + 12, p + 4,
-                                                  torch.cuda.current_stream(out.device).cuda_stream)
+                    _lib.unscale_clip_coefficient(table._aw4_rows, p + 8, max_norm, p, p + 12, p + 4,
+                                                  _raw_stream(out.device.index))
         elif torch.compiler.is_compiling():
             _ops.clip_coefficient_(grads, out, table, max_norm)
         else:  # the operator's dispatch over every gradient costs more than the call (see _launch)
-            with torch.cuda.device(out.device):
+            with _current_device(out.device.index):
                 p = out.data_ptr()
-                _lib.clip_coefficient(table.numpy().view(_lib.TENSOR), max_norm, p, p + 12,
-                                      torch.cuda.current_stream(out.device).cuda_stream)
+                _lib.clip_coefficient(table._aw4_rows, max_norm, p, p + 12, _raw_stream(out.device.index))
         total = out[0].to(result_dtype)
         if error_if_nonfinite and bool(torch.logical_or(total.isnan(), total.isinf())):
             raise RuntimeError(
@@ -826,6 +835,11 @@ class QuantizedAdamW(Optimizer):
         without gradients."""
         if self._grad_clip is not None:
             raise RuntimeError("a gradient clip is already pending: call step() before clipping again")
+        if self._clip_plan is not None and not torch.compiler.is_compiling():
+            prepared = self._clip_plan.prepare(self)
+            if prepared is not None:
+                return prepared
+        self._clip_plan = None
         params = [p for group in self.param_groups for p in group["params"] if p.grad is not None]
         if not params:
             return None
@@ -850,7 +864,10 @@ class QuantizedAdamW(Optimizer):
         for g in grads[1:]:
             if g.dtype != result_dtype:
                 result_dtype = torch.float32  # torch.stack promotes the per-tensor norms
-        return grads, torch.from_numpy(table.view(np.uint8)), out, result_dtype
+        table_t = _table_tensor(table)
+        if all(p.grad is g for p, g in zip(params, grads)):
+            self._clip_plan = _ClipPlan(grads, table, table_t, result_dtype)
+        return grads, table_t, out, result_dtype
 
     @torch.compiler.disable
     def _set_grad_clip(self, out: torch.Tensor, flags: int) -> None:
@@ -1349,6 +1366,47 @@ _SMALL_PLAN = 16
 _REPEAT_STEP, _REPEAT_INT = itertools.repeat("step"), itertools.repeat(int)
 
 
+class _ClipPlan:
+    """The last clip's table, reused while the gradients it describes only move: each call checks every
+    gradient's dtype, size, device and layout against the rows, and rewrites their addresses."""
+
+    __slots__ = ("dtypes", "numels", "index", "device", "vec", "table", "table_t", "result_dtype", "addresses")
+
+    def __init__(self, grads, table: np.ndarray, table_t: torch.Tensor, result_dtype):
+        self.dtypes = [g.dtype for g in grads]
+        self.numels = [g.numel() for g in grads]
+        self.device = grads[0].device
+        self.index = self.device.index
+        self.vec = np.array([4 * g.element_size() for g in grads], dtype=np.uint64)
+        self.table, self.table_t, self.result_dtype = table, table_t, result_dtype
+        self.addresses = [g.data_ptr() for g in grads]  # what the table holds
+
+    def prepare(self, opt: "QuantizedAdamW"):
+        """As ``_prepare_clip``, or None if the gradients are not the table's."""
+        strided, index = torch.strided, self.index
+        grads, addresses = [], []
+        n, i = len(self.numels), 0
+        for group in opt.param_groups:
+            for p in group["params"]:
+                g = p.grad
+                if g is None:
+                    continue
+                if (i >= n or g.dtype is not self.dtypes[i] or g.numel() != self.numels[i] or g.layout is not strided
+                        or g.get_device() != index or not g.is_contiguous()):
+                    return None
+                grads.append(g)
+                addresses.append(g.data_ptr())
+                i += 1
+        if i != n:
+            return None
+        if addresses != self.addresses:
+            a = np.array(addresses, dtype=np.uint64)
+            self.table["grad"] = a
+            self.table["flags"] = np.where(a % self.vec == 0, _lib.TENSOR_VEC_ALIGNED, 0)
+            self.addresses = addresses
+        return grads, self.table_t, torch.empty(4, dtype=torch.float32, device=self.device), self.result_dtype
+
+
 class _PlanDevice:
     """One device's part of a launch plan: its table (rows with every address filled in) and
     the views and per-row facts its per-step refresh needs."""
@@ -1357,7 +1415,8 @@ class _PlanDevice:
                  "gbytes", "gbytes_list", "pvec", "pvec_list", "gvec", "gvec_list", "fields", "words",
                  "m2_sr", "seed_cols", "offset_cols", "grad_col", "qrows", "qsel", "qrows_any", "la_rows", "la_next",
                  "f64", "f64_rows", "refs", "table_t", "refs_t", "scale_ptr", "scale_ref", "buf", "row_plans",
-                 "rows", "index", "bump", "gchecked")
+                 "rows", "index", "bump", "gchecked", "garray", "gflags", "gflags_of", "classes", "row_class", "draws",
+                 "qrows_list")
 
     def __init__(self, table: np.ndarray, params, written, entries, lo, hi, ranges, refs: np.ndarray):
         n = len(params)
@@ -1401,6 +1460,13 @@ class _PlanDevice:
         self.index = self.device.index
         self.bump = self.params + self.written  # what an eager launch writes in place
         self.gchecked = None  # the gradient addresses whose overlap check last passed
+        self.garray = None    # the same as an array (larger plans), and the flags and table column made of them
+        self.gflags = self.gflags_of = None
+        # rows by what their step constants depend on besides the step count, and the rows that draw
+        self.classes = list(dict.fromkeys((e[1], e[2]) for e in entries))
+        self.row_class = [self.classes.index((e[1], e[2])) for e in entries]
+        self.draws = [(i, moment, stream, e[4]) for i, e in enumerate(entries) for moment, stream in e[3]]
+        self.qrows_list = self.qrows.tolist()
         # small plans write each row's per-step fields in place (struct.pack_into at the row's
         # offsets): per row whether m2 takes the update-SR constants, is float64, is lookahead
         self.buf = memoryview(table.view(np.uint8)).cast("B")
@@ -1592,10 +1658,13 @@ class _LaunchPlan:
                                 return None
                     dev.gchecked = g0
             else:
-                g0 = np.array(g0, dtype=np.int64)
-                g1 = g0 + dev.gbytes
-                if bool(((dev.lo < g1[:, None]) & (g0[:, None] < dev.hi)).any()):
-                    return None
+                if g0 != dev.gchecked:
+                    a0 = np.array(g0, dtype=np.int64)
+                    a1 = a0 + dev.gbytes
+                    if bool(((dev.lo < a1[:, None]) & (a0[:, None] < dev.hi)).any()):
+                        return None
+                    dev.gchecked, dev.garray = g0, a0
+                g0 = (g0, dev.garray)
             out.append(g0)
         return out
 
@@ -1645,34 +1714,49 @@ class _LaunchPlan:
                         _PACK_RNG(buf, off + _OFF_RNG[moment], stream.seed, stream.take(numel))
                 ks = None
             else:
-                ks = []  # constants index of each row
+                # one step count for every row (as training has it): a constants entry per row class;
+                # else one per row
+                states = dev.states
+                step = states[0]["step"] + 1
+                if all(map(operator.eq, map(dict.get, states, _REPEAT_STEP), itertools.repeat(step - 1))):
+                    for state in states:
+                        state["step"] = step
+                    of_class = [constants_of(gi, step, m2_scheme) for gi, m2_scheme in dev.classes]
+                    ks = of_class * len(entries) if len(of_class) == 1 else list(map(of_class.__getitem__, dev.row_class))
+                else:
+                    ks = []  # constants index of each row
+                    for state, gi, m2_scheme, sr, numel in entries:
+                        step = state["step"] + 1
+                        state["step"] = step
+                        ks.append(constants_of(gi, step, m2_scheme))
                 seeds, offsets = dev.seed_cols, dev.offset_cols
-                for i, (state, gi, m2_scheme, sr, numel) in enumerate(entries):
-                    step = state["step"] + 1
-                    state["step"] = step
-                    ks.append(constants_of(gi, step, m2_scheme))
-                    for moment, stream in sr:
-                        seeds[moment][i] = stream.seed
-                        offsets[moment][i] = stream.take(numel)
+                for i, moment, stream, numel in dev.draws:
+                    seeds[moment][i] = stream.seed
+                    offsets[moment][i] = stream.take(numel)
                 # the flags word and the seven fp32 step constants (bit patterns), and the m2
                 # update-SR constants of the rows whose m2 is quantized
-                one = ks.count(ks[0]) == len(ks)
-                if one:
-                    dev.words[:] = consts[ks[0]].words()
+                index = None
+                words = [c.words_bytes() for c in consts]
+                if words.count(words[0]) == len(words):  # every class the same (one group): one broadcast
+                    dev.words[:] = consts[0].words()
                 else:
                     index = np.array(ks, dtype=np.intp)
                     dev.words[:] = np.stack([c.words() for c in consts])[index]
-                dev.words[:, 0] |= (np.where(dev.pvec & (g0 % dev.gvec == 0), _lib.TENSOR_VEC_ALIGNED, 0)
-                                    | extra).astype(np.uint32)
+                g0_list, g0 = g0
+                if g0_list != dev.gflags_of:
+                    dev.gflags = np.where(dev.pvec & (g0 % dev.gvec == 0), _lib.TENSOR_VEC_ALIGNED, 0).astype(np.uint32)
+                    dev.grad_col[:] = g0
+                    dev.gflags_of = g0_list
+                dev.words[:, 0] |= dev.gflags | np.uint32(extra) if extra else dev.gflags
                 if dev.qrows_any:
-                    if one:
-                        dev.m2_sr[dev.qsel] = consts[ks[0]].m2_sr()
+                    if len({ks[i] for i in dev.qrows_list}) == 1:
+                        dev.m2_sr[dev.qsel] = consts[ks[dev.qrows_list[0]]].m2_sr()
                     else:
+                        index = np.array(ks, dtype=np.intp) if index is None else index
                         dev.m2_sr[dev.qrows] = np.stack([c.m2_sr() for c in consts])[index[dev.qrows]]
                 if len(dev.f64_rows):
                     dev.f64[dev.f64_rows] = [(consts[ks[i]].decay_f64, consts[ks[i]].step_coef_f64)
                                              for i in dev.f64_rows.tolist()]
-                dev.grad_col[:] = g0
             if len(dev.la_rows):
                 # the lookahead fields, by the full path's arithmetic (Python floats)
                 la = []
