@@ -365,6 +365,8 @@ constexpr int kNumSpecialised = kResearchVariant;
 // a CU), and the grid covers every tile at kCodecTiles per wave, which share the table fill.
 // Measured, nf4, us encode / decode of 2^24 values: 28 / 28 with all tables and a grid of eight
 // workgroups per CU, 14.9 / 13.4 so (5.1 / 5.7 TB/s); 2^27 values 112 / 124 us (5.4 / 4.9 TB/s).
+// Decode's stores are non-temporal, as the other kernels' are: dirty lines left in the L2s were written
+// back while the next launch waited (the pair, 2^24 values: 35.3 -> 27.6 us, 5.5 TB/s).
 // Encoding nf4_sr is bound by its draws (26.7 us).
 constexpr int kCodecTiles = 4;
 
@@ -460,7 +462,8 @@ __global__ void __launch_bounds__(kThreads) dequantize_kernel(aw4_moment M, int6
             const int64_t e = e0 + 256 * q;
             float m[4];
             decode4(dec, w[q], scale[q], m);
-            if (e < numel) *(gptr<f32x4>)gaddr<float>((uint64_t)(out + e)) = f32x4{m[0], m[1], m[2], m[3]};
+            if (e < numel)
+                __builtin_nontemporal_store(f32x4{m[0], m[1], m[2], m[3]}, (gptr<f32x4>)gaddr<float>((uint64_t)(out + e)));
         }
     }
 }
