@@ -412,7 +412,8 @@ struct BlockScales {
 template <int KIND, bool kNonNeg, class Values>
 __device__ __forceinline__ bool encode_quick(const aw4_moment& M, const MomentTables& L, int64_t blk0, int grp, int j,
                                              const Values& vals, float s, float y, const UsrBlock& ub, bool eden,
-                                             bool floor0, float (&acc_xx)[4], float (&acc_xl)[4], BlockScratch sc) {
+                                             bool floor0, uint64_t tile_counter, float (&acc_xx)[4],
+                                             float (&acc_xl)[4], BlockScratch sc) {
     uint64_t unsure = 0;  // lanes (bits) with a value the quick test leaves open
     uint32_t rw[12];
 #pragma unroll
@@ -428,7 +429,7 @@ __device__ __forceinline__ bool encode_quick(const aw4_moment& M, const MomentTa
         }
         if constexpr (KIND != K_RTN) {
             float u[4];
-            if (q < 3) philox_tile_call(M.rng_seed, (M.rng_offset >> 7) + (uint64_t)blk0, grp, j, q, &rw[4 * q]);
+            if (q < 3) philox_tile_call_one_hi(M.rng_seed, tile_counter, grp, j, q, &rw[4 * q]);
             lane_fields4(&rw[3 * q], u);
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -500,8 +501,15 @@ __device__ __forceinline__ BlockScales encode_block(const aw4_moment& M, const M
     float acc_xx[4] = {0.0f, 0.0f, 0.0f, 0.0f}, acc_xl[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     bool settled = false;
     if constexpr (kQuick) {
-        if (__builtin_expect(wave_fast & ((M.flags & AW4_MOMENT_EXT_DRAWS) == 0), 1))
-            settled = encode_quick<KIND, kNonNeg>(M, L, blk0, grp, j, vals, s, y, ub, eden, floor0, acc_xx, acc_xl, sc);
+        bool quick = wave_fast & ((M.flags & AW4_MOMENT_EXT_DRAWS) == 0);
+        uint64_t tile_counter = 0;
+        if constexpr (KIND != K_RTN) {
+            tile_counter = philox_tile_counter((M.rng_offset >> 7) + (uint64_t)blk0);
+            quick = quick & philox_tile_one_hi(tile_counter);
+        }
+        if (__builtin_expect(quick, 1))
+            settled = encode_quick<KIND, kNonNeg>(M, L, blk0, grp, j, vals, s, y, ub, eden, floor0, tile_counter, acc_xx,
+                                                  acc_xl, sc);
         if (__builtin_expect(!settled, 0)) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) acc_xx[t] = acc_xl[t] = 0.0f;

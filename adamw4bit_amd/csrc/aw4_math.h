@@ -171,13 +171,17 @@ __device__ __forceinline__ float block_sum_cross(const float (&acc)[4]) {
 // its 16 uniforms from three Philox calls, every output bit used once.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t k0, uint32_t k1,
-                                              uint32_t* out) {
-    uint32_t c2 = 0u, c3 = 0u;
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u, kPhiloxM1 = 0xCD9E8D57u;  // multipliers
+constexpr uint32_t kPhiloxW0 = 0x9E3779B9u, kPhiloxW1 = 0xBB67AE85u;  // key increments
+
+// kRounds rounds of the words c0..c3, the first with key (k0, k1).
+template <int kRounds>
+__device__ __forceinline__ void philox_rounds(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
+                                              uint32_t k1, uint32_t* out) {
 #pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        const uint64_t p0 = (uint64_t)0xD2511F53u * c0;
-        const uint64_t p1 = (uint64_t)0xCD9E8D57u * c2;
+    for (int r = 0; r < kRounds; ++r) {
+        const uint64_t p0 = (uint64_t)kPhiloxM0 * c0;
+        const uint64_t p1 = (uint64_t)kPhiloxM1 * c2;
         // three-input exclusive or in one v_bitop3_b32 (truth table 0x96, symmetric in its inputs)
         const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);
         const uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
@@ -185,8 +189,8 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
         c3 = (uint32_t)p0;
         c0 = n0;
         c2 = n2;
-        k0 += 0x9E3779B9u;
-        k1 += 0xBB67AE85u;
+        k0 += kPhiloxW0;
+        k1 += kPhiloxW1;
     }
     out[0] = c0;
     out[1] = c1;
@@ -196,7 +200,7 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t
 
 // Philox(counter = ctr, key = seed): four output words.
 __device__ __forceinline__ void philox_call(uint64_t seed, uint64_t ctr, uint32_t* w) {
-    philox4x32_10((uint32_t)ctr, (uint32_t)(ctr >> 32), (uint32_t)seed, (uint32_t)(seed >> 32), w);
+    philox_rounds<10>((uint32_t)ctr, (uint32_t)(ctr >> 32), 0u, 0u, (uint32_t)seed, (uint32_t)(seed >> 32), w);
 }
 
 // Call r (0..2) of lane j in position group B: words 4r .. 4r+3 of the lane's 384-bit string.
@@ -204,18 +208,40 @@ __device__ __forceinline__ void philox_lane_call(uint64_t seed, uint64_t group, 
     philox_call(seed, group * 24u + (uint64_t)(3 * j + r), w);
 }
 
-// The same call for block grp of a wave tile whose first block is position group g0 (wave-uniform):
-// counter 24 (g0 + grp) + 3 j + r = 24 g0 + 3 (8 grp + j) + r, so the 64-bit product is the
-// wave's (a scalar one) and each lane adds its small constant.
-__device__ __forceinline__ void philox_tile_call(uint64_t seed, uint64_t g0, int grp, int j, int r, uint32_t* w) {
-    // The product in scalar registers: read as the first lane's (g0 is the wave tile's, the same in
-    // every lane), and held there by an empty asm statement, so that each lane's counter is one
-    // 64-bit add rather than two 64-bit vector multiply-adds.
+// The counter of the first call of a wave tile whose first block is position group g0 (wave-uniform):
+// lane j's call r in block grp has counter 24 (g0 + grp) + 3 j + r = 24 g0 + 3 (8 grp + j) + r.  The
+// 64-bit product is in scalar registers: read as the first lane's (g0 is the wave tile's, the same in
+// every lane), and held there by an empty asm statement, so that a lane's counter is an addition rather
+// than two 64-bit vector multiply-adds.
+__device__ __forceinline__ uint64_t philox_tile_counter(uint64_t g0) {
     const uint64_t prod = g0 * 24u;
     uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)prod);
     uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(prod >> 32));
     asm("" : "+s"(lo), "+s"(hi));
-    philox_call(seed, ((uint64_t)hi << 32 | lo) + (uint32_t)(24 * grp + 3 * j + r), w);
+    return (uint64_t)hi << 32 | lo;
+}
+
+__device__ __forceinline__ void philox_tile_call(uint64_t seed, uint64_t g0, int grp, int j, int r, uint32_t* w) {
+    philox_call(seed, philox_tile_counter(g0) + (uint32_t)(24 * grp + 3 * j + r), w);
+}
+
+// Whether the tile's 192 counters (8 blocks of 24) share their upper word: all but one tile in 2^32 / 192.
+__device__ __forceinline__ bool philox_tile_one_hi(uint64_t tile_counter) {
+    return (uint32_t)tile_counter <= 0xffffffffu - 191u;
+}
+
+// The call of such a tile: the upper word stays the wave's scalar, and with it the first round's c0 and one
+// of the second round's products (18 vector products instead of 19, two-input exclusive ors in those rounds
+// and a 32-bit counter addition).
+__device__ __forceinline__ void philox_tile_call_one_hi(uint64_t seed, uint64_t tile_counter, int grp, int j, int r,
+                                                        uint32_t* w) {
+    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+    const uint64_t p0 = (uint64_t)kPhiloxM0 * ((uint32_t)tile_counter + (uint32_t)(24 * grp + 3 * j + r));
+    const uint64_t s0 = (uint64_t)kPhiloxM0 * ((uint32_t)(tile_counter >> 32) ^ k0);  // round 2, scalar
+    const uint64_t p1 = (uint64_t)kPhiloxM1 * ((uint32_t)(p0 >> 32) ^ k1);            // round 2
+    philox_rounds<8>((uint32_t)(p1 >> 32) ^ (k0 + kPhiloxW0), (uint32_t)p1,
+                     ((uint32_t)(s0 >> 32) ^ (k1 + kPhiloxW1)) ^ (uint32_t)p0, (uint32_t)s0, k0 + 2 * kPhiloxW0,
+                     k1 + 2 * kPhiloxW1, w);
 }
 
 // Fields 4q .. 4q+3 of a lane's string (words 3q .. 3q+2), as exact floats in [0, 2^24):
