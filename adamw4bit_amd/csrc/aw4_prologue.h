@@ -75,7 +75,7 @@ template <int G, bool kUnscale>
 __device__ __forceinline__ double sq4(uint64_t grad, int64_t e, bool vec, float u, bool& bad) {
     uint32_t w[4];
     float f[4];
-    load_words<G>(grad, e, vec, w);
+    load_words<G, true>(grad, e, vec, w);
     words_to_f32<G>(w, f);
     double s = 0.0;
 #pragma unroll

@@ -33,13 +33,14 @@ struct StepHeader {
 // 4-value vector access (streaming: each byte is touched once per step)
 // ---------------------------------------------------------------------------
 
-// Raw 32-bit words of 4 values: fp32 values, or 2 words of packed 16-bit values.
-template <int D>
+// Raw 32-bit words of 4 values: fp32 values, or 2 words of packed 16-bit values.  kKeep: through the caches
+// (values that the next launch reads again), not past them.
+template <int D, bool kKeep = false>
 __device__ __forceinline__ void load_words(uint64_t base, int64_t e, bool vec, uint32_t* w) {
     if constexpr (D == D_F32) {
         const gptr<const float> p = gaddr<const float>(base) + e;
         if (vec) {
-            const u32x4 v = __builtin_nontemporal_load((gptr<const u32x4>)p);
+            const u32x4 v = kKeep ? *(gptr<const u32x4>)p : __builtin_nontemporal_load((gptr<const u32x4>)p);
             w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
         } else {
 #pragma unroll
@@ -48,7 +49,7 @@ __device__ __forceinline__ void load_words(uint64_t base, int64_t e, bool vec, u
     } else {
         const gptr<const uint16_t> p = gaddr<const uint16_t>(base) + e;
         if (vec) {
-            const u32x2 v = __builtin_nontemporal_load((gptr<const u32x2>)p);
+            const u32x2 v = kKeep ? *(gptr<const u32x2>)p : __builtin_nontemporal_load((gptr<const u32x2>)p);
             w[0] = v.x; w[1] = v.y;
         } else {
             w[0] = (uint32_t)p[0] | ((uint32_t)p[1] << 16);
