@@ -713,7 +713,10 @@ struct StagingSlot {
     const void* host_dev = nullptr;  // the device's address of `host`
     void* dev = nullptr;             // device copy the kernels read
     size_t cap = 0;
-    uint32_t* tickets = nullptr;     // the norm pass's workgroup counters, behind `dev`: zero outside its launches
+    // The norm pass's workgroup counters, behind `dev`, zero outside its launches: the gradients', and the
+    // segment groups'.
+    uint32_t* tickets = nullptr;
+    uint32_t* ticket_groups = nullptr;
     hipEvent_t done = nullptr;
     bool pending = false;
 };
@@ -1019,10 +1022,13 @@ int acquire_slot(DeviceState* ds, size_t bytes, StagingSlot** out) {
         void* mapped = nullptr;
         AW4_HIP_CHECK(hipHostGetDevicePointer(&mapped, slot.host, 0));
         slot.host_dev = mapped;
-        // The counters: one per gradient and one more, of a pass that keeps 8 bytes per gradient in `dev`.
-        const std::vector<uint32_t> zero(cap / 8 + 1, 0u);
+        // The counters: one per gradient and one more, and those of the segment groups, of a pass that keeps
+        // 8 bytes per gradient and per segment in `dev`.
+        const size_t words = (cap / 8 + 1 + kNormGroupStride - 1) / kNormGroupStride * kNormGroupStride;
+        const std::vector<uint32_t> zero(words + (size_t)norm_group_words((int64_t)(cap / 8)), 0u);
         AW4_HIP_CHECK(hipMalloc(&slot.dev, cap + zero.size() * sizeof(uint32_t)));
         slot.tickets = (uint32_t*)((char*)slot.dev + cap);
+        slot.ticket_groups = slot.tickets + words;
         AW4_HIP_CHECK(hipMemcpy(slot.tickets, zero.data(), zero.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
         slot.cap = cap;
     }
@@ -1445,6 +1451,7 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     h->partials = (uint64_t)slot->dev + scratch_at;
     h->norm_sq = h->partials + sizeof(double) * (uint64_t)segments;
     h->tickets = (uint64_t)slot->tickets;
+    h->groups = (uint64_t)slot->ticket_groups;
     h->norm_out = (uint64_t)norm_out;
     h->coef_out = (uint64_t)coef_out;
     if (unscale) {

@@ -130,7 +130,9 @@ def test_codec_sizes_match_oracle(mode, eden, blocks):
 @pytest.mark.parametrize("sizes", [[1], [3], [8191, 8193, 5], [4096 * 4096], [1 << 18] * 9 + [1000001],
                                    [257 * (i % 7 + 1) for i in range(156)],   # the most rows launch arguments hold
                                    [257 * (i % 7 + 1) for i in range(157)],   # one more: a staged table
-                                   [40_000_003, 11, 30_000_000]])
+                                   [40_000_003, 11, 30_000_000],
+                                   # runs of 32 segments: more and fewer than one, parts of one at both ends
+                                   [8192 * 33, 5, 8192 * 40 + 1, 8192 * 32, 8192 * 70 - 3]])
 def test_clip_norm_sizes(sizes, dtype):
     """The norm pass over segments of 2^13 to 2^15 values, cut ones, many gradients and one; twice, since
     its counters must be zero again.  The same gradients one value off their alignment, too."""
