@@ -3,8 +3,8 @@
 ``python -m adamw4bit_amd.build`` compiles ``csrc/fused_step.hip`` with hipcc
 (no GPU needed: hipcc cross-compiles for ``--offload-arch=gfx950``) twice: the
 main object, and one with ``AW4_SCHED_ILP_TU`` that holds only the bf16
-update-SR kernels, scheduled by LLVM's max-ilp strategy; one link makes the
-library.  It lands next to this file so it travels with the source tree.
+update-SR, the fp16 round-to-nearest and the code-storing lookahead kernels,
+scheduled by LLVM's max-ilp strategy; one link makes the library.  It lands next to this file so it travels with the source tree.
 
 Flags that are part of the numerical contract:
   -ffp-contract=off   no implicit multiply-add fusion; the kernel writes each
@@ -42,8 +42,8 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found (set HIPCC or install ROCm)")
 
 
-# The second object: the same source with AW4_SCHED_ILP_TU, which emits only the bf16
-# update-SR kernels, scheduled by LLVM's max-ilp strategy (the source says why).
+# The second object: the same source with AW4_SCHED_ILP_TU, which emits only the kernels that
+# gain from LLVM's max-ilp strategy (the source says which and why).
 ILP_FLAGS = ("-DAW4_SCHED_ILP_TU", "-mllvm", "-amdgpu-sched-strategy=max-ilp")
 
 

@@ -248,17 +248,31 @@ values_kernel_inline(const InlineArgs a) {
 
 }  // namespace
 
-// The bf16 update-SR kernels (ZIP-SR and its nf4_sr head) come from a second compile of this file, with
-// AW4_SCHED_ILP_TU defined and LLVM's max-ilp machine scheduler (-mllvm -amdgpu-sched-strategy=max-ilp);
-// that object holds nothing else.  Bound by their instruction issue, the bf16 kernels ran 1.2-1.5% faster
-// under it, while ZE-EDEN spilled (4% slower).  Since the update-SR encode is one stretch of code
-// (encode_quick), the fp32 one and the EDEN-m2 ablation spill under it too (37 and 4 registers) and keep
-// the default scheduler.  The main object declares these kernels and launches them through the variant
-// table.
+// The bf16 update-SR kernels (ZIP-SR and its nf4_sr head), the fp16 round-to-nearest ones and the
+// code-storing lookahead ones come from a second compile of this file, with AW4_SCHED_ILP_TU defined and
+// LLVM's max-ilp machine scheduler (-mllvm -amdgpu-sched-strategy=max-ilp); that object holds nothing else.
+// Bound by their instruction issue, they run faster under it: the bf16 update-SR ones 1.2-1.5%; one
+// Llama-3-8B layer under the proxy lookahead fp32 735.7 -> 714.4 us, bf16 724.3 -> 690.4 us; under ZE-EDEN
+// fp16 385.9 -> 383.0 us, sdyn4 / dyn4 fp16 373.0 -> 370.9 us.  The bf16 round-to-nearest kernels gain
+// nothing beyond a run's spread (374.4 and 373.7 us), and ZE-EDEN fp32 spilled (4% slower).  Since the
+// update-SR encode is one stretch of code (encode_quick), the fp32 one and the EDEN-m2 ablation spill under
+// it too (37 and 4 registers); all of these keep the default scheduler.  The main object declares these
+// kernels and launches them through the variant table.
 namespace aw4_ilp {
 template <int M1K, int M2K, int D>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
 step_kernel_4w(const aw4::StepHeader* __restrict__ hdr, const aw4::Tables* __restrict__ tables)
+#ifdef AW4_SCHED_ILP_TU
+{
+    step_body<M1K, M2K, D>(hdr, tables);
+}
+#else
+    ;
+#endif
+
+template <int M1K, int M2K, int D>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
+step_kernel_3w(const aw4::StepHeader* __restrict__ hdr, const aw4::Tables* __restrict__ tables)
 #ifdef AW4_SCHED_ILP_TU
 {
     step_body<M1K, M2K, D>(hdr, tables);
@@ -297,6 +311,11 @@ constexpr int kAnyResearch = mspec(K_ANY, AW4_MOMENT_SAMPLED_READ);
 template __global__ void aw4_ilp::step_kernel_4w<kRtn, kUsrGuarded, D_BF16>(const aw4::StepHeader*, const aw4::Tables*);
 template __global__ void aw4_ilp::step_kernel_4w<kSsrGuarded, kUsrGuarded, D_BF16>(const aw4::StepHeader*,
                                                                                    const aw4::Tables*);
+template __global__ void aw4_ilp::step_kernel_4w<kRtn, kRtnEden, D_F16>(const aw4::StepHeader*, const aw4::Tables*);
+template __global__ void aw4_ilp::step_kernel_4w<kRtn, kRtn, D_F16>(const aw4::StepHeader*, const aw4::Tables*);
+template __global__ void aw4_ilp::step_kernel_3w<kRtn, kLaStore, D_F32>(const aw4::StepHeader*, const aw4::Tables*);
+template __global__ void aw4_ilp::step_kernel_3w<kRtn, kLaStore, D_BF16>(const aw4::StepHeader*, const aw4::Tables*);
+template __global__ void aw4_ilp::step_kernel_3w<kRtn, kLaStore, D_F16>(const aw4::StepHeader*, const aw4::Tables*);
 #else
 
 struct KernelVariant {
@@ -314,6 +333,7 @@ struct KernelVariant {
     {M1, M2, D, (const void*)&step_kernel_4w<M1, M2, D>, (const void*)&step_kernel_inline_4w<M1, M2, D>}
 // the max-ilp instances of the second object (their small-step instances stay in this one)
 #define AW4_VARIANT_ILP(M1, M2, D) {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, nullptr}
+#define AW4_VARIANT_ILP_3W(M1, M2, D) {M1, M2, D, (const void*)&aw4_ilp::step_kernel_3w<M1, M2, D>, nullptr}
 #define AW4_VARIANT_ILP_I4W(M1, M2, D) \
     {M1, M2, D, (const void*)&aw4_ilp::step_kernel_4w<M1, M2, D>, (const void*)&step_kernel_inline_4w<M1, M2, D>}
 // launches of fp32-state tensors of one dtype
@@ -332,16 +352,16 @@ const KernelVariant kVariants[] = {
     AW4_VARIANT(kSsrGuarded, kUsrGuarded, D_F32), AW4_VARIANT_ILP(kSsrGuarded, kUsrGuarded, D_BF16),
     AW4_VARIANT(kRtn, kFp32, D_F32),              AW4_VARIANT(kRtn, kFp32, D_BF16),
     AW4_VARIANT(kRtn, kUsrGuardedEden, D_F32),    AW4_VARIANT_4W(kRtn, kUsrGuardedEden, D_BF16),
-    AW4_VARIANT_4W(kRtn, kRtnEden, D_F16),        AW4_VARIANT_4W(kRtn, kUsrGuarded, D_F16),
+    AW4_VARIANT_ILP(kRtn, kRtnEden, D_F16),       AW4_VARIANT_4W(kRtn, kUsrGuarded, D_F16),
     AW4_VARIANT_4W(kSsrGuarded, kUsrGuarded, D_F16),
     AW4_VARIANT(kRtn, kFp32, D_F16),              AW4_VARIANT_4W(kRtn, kUsrGuardedEden, D_F16),
     AW4_VARIANT_4W(kRtn, kRtn, D_F32),            AW4_VARIANT_4W(kRtn, kRtn, D_BF16),
-    AW4_VARIANT_4W(kRtn, kRtn, D_F16),
+    AW4_VARIANT_ILP(kRtn, kRtn, D_F16),
     AW4_VARIANT_VALUES(D_F32), AW4_VARIANT_VALUES(D_BF16), AW4_VARIANT_VALUES(D_F16),
     AW4_VARIANT(kRtn, kUsrRead, D_F32),           AW4_VARIANT(kRtn, kUsrReadEden, D_F32),
-    AW4_VARIANT(kRtn, kLaStore, D_F32),           AW4_VARIANT_3W(kRtn, kLaPending, D_F32),
+    AW4_VARIANT_ILP_3W(kRtn, kLaStore, D_F32),    AW4_VARIANT_3W(kRtn, kLaPending, D_F32),
     AW4_VARIANT(kRtn, kUsrRead, D_BF16),          AW4_VARIANT(kRtn, kUsrRead, D_F16),
-    AW4_VARIANT_3W(kRtn, kLaStore, D_BF16),       AW4_VARIANT_3W(kRtn, kLaStore, D_F16),
+    AW4_VARIANT_ILP_3W(kRtn, kLaStore, D_BF16),   AW4_VARIANT_ILP_3W(kRtn, kLaStore, D_F16),
     AW4_VARIANT_2W(K_ANY, kAnyResearch, D_ANY),
     AW4_VARIANT(K_ANY, K_ANY, D_ANY),
 };
@@ -353,6 +373,7 @@ const KernelVariant kVariants[] = {
 #undef AW4_VARIANT_I
 #undef AW4_VARIANT_I4W
 #undef AW4_VARIANT_ILP
+#undef AW4_VARIANT_ILP_3W
 #undef AW4_VARIANT_ILP_I4W
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 constexpr int kGenericVariant = kNumVariants - 1;
