@@ -55,7 +55,10 @@
 // second compile of this file, AW4_SCHED_ILP_TU below, emits kernels and nothing else.)
 #ifndef AW4_SCHED_ILP_TU
 static __device__ __align__(256) uint8_t g_tables_mem[sizeof(aw4::Tables) + AW4_NUM_LUTS * sizeof(aw4::LinTable)];
-static __device__ __align__(256) uint8_t scratch[AW4_NOALLOC_TABLE_BYTES];
+// Launch tables of AW4_NOALLOC_TABLE_BYTES, and beyond them the header and the padding of every launch after
+// the first that such a table can split into: whether a call fits depends on its rows alone.
+constexpr size_t kNoallocGroupBytes = 1 << 17;
+static __device__ __align__(256) uint8_t scratch[AW4_NOALLOC_TABLE_BYTES + kNoallocGroupBytes];
 #endif
 
 namespace {
@@ -1070,6 +1073,15 @@ struct StepLaunch {
     size_t bytes = 0;
 };
 
+// Bytes of the launch table of n tensors (header, rows, tile starts), and with its padding to 256 bytes.
+size_t table_bytes(size_t n) { return sizeof(StepHeader) + sizeof(aw4_tensor) * n + sizeof(int64_t) * (n + 1); }
+size_t padded_table_bytes(size_t n) { return (table_bytes(n) + 255) & ~(size_t)255; }
+
+// A step has at most one launch for each specialised variant, the two codebooks of a specialised first
+// moment and the second moment's five and floored dyn4, and the two generic ones.
+static_assert((12 * kNumSpecialised + 2) * (sizeof(StepHeader) + sizeof(int64_t) + 255) <= kNoallocGroupBytes,
+              "the table area of aw4_fused_step_noalloc holds every split of a call that fits it unsplit");
+
 // Validate the rows and plan the launches (no device work, no lock needed).
 int prepare_step(const aw4_tensor* tensors, int32_t count, StepLaunch& sl) {
     if (count < 0 || (count > 0 && !tensors)) return set_error(AW4_EINVAL, "aw4_fused_step: bad tensor list");
@@ -1084,9 +1096,8 @@ int prepare_step(const aw4_tensor* tensors, int32_t count, StepLaunch& sl) {
     sl.grid.assign(sl.plan.size(), 0);
     sl.bytes = 0;
     for (size_t g = 0; g < sl.plan.size(); ++g) {
-        const size_t n = sl.plan[g].members.size();
         sl.offset[g] = sl.bytes;
-        sl.bytes += (sizeof(StepHeader) + sizeof(aw4_tensor) * n + sizeof(int64_t) * (n + 1) + 255) & ~(size_t)255;
+        sl.bytes += padded_table_bytes(sl.plan[g].members.size());
     }
     return AW4_OK;
 }
@@ -1201,11 +1212,8 @@ int launch_step(const StepLaunch& sl, const char* dev_base, const Tables* tables
     return AW4_OK;
 }
 
-// Bytes of group g's launch table (header, rows, tile starts; without the 256-byte padding).
-size_t group_table_bytes(const StepLaunch& sl, size_t g) {
-    const size_t n = sl.plan[g].members.size();
-    return sizeof(StepHeader) + sizeof(aw4_tensor) * n + sizeof(int64_t) * (n + 1);
-}
+// Bytes of group g's launch table, without the padding.
+size_t group_table_bytes(const StepLaunch& sl, size_t g) { return table_bytes(sl.plan[g].members.size()); }
 
 // Whether every group can take its table in its launch's arguments.
 bool fits_inline(const StepLaunch& sl) {
@@ -1331,11 +1339,13 @@ int aw4_fused_step_noalloc(const aw4_tensor* tensors, int32_t count, void* strea
     StepLaunch sl;
     int rc = prepare_step(tensors, count, sl);
     if (rc || sl.plan.empty()) return rc;
-    if (sl.bytes > (size_t)AW4_NOALLOC_TABLE_BYTES)
+    // By the rows, not by how many launches they split into (the area has room for those, kNoallocGroupBytes).
+    const size_t unsplit = padded_table_bytes((size_t)count);
+    if (unsplit > (size_t)AW4_NOALLOC_TABLE_BYTES || sl.bytes > sizeof(scratch))
         return set_error(AW4_EINVAL,
                          "aw4_fused_step_noalloc: the launch tables of %d tensors need %zu bytes, more than its "
                          "%d-byte table area (use aw4_fused_step)",
-                         count, sl.bytes, AW4_NOALLOC_TABLE_BYTES);
+                         count, std::max(unsplit, sl.bytes), AW4_NOALLOC_TABLE_BYTES);
     std::lock_guard<std::mutex> lock(g_mutex);
     DeviceState* ds = nullptr;
     rc = device_state(&ds);

@@ -193,9 +193,10 @@ int aw4_fused_step(const aw4_tensor* tensors, int32_t count, void* stream);
  * the reference (whose step is Python).  Same arguments, checks, kernels and results as
  * aw4_fused_step, but it calls no hipMalloc, hipFree or other allocating routine: the launch
  * tables (the step's only device memory besides the caller's tensors) go to a fixed area of
- * AW4_NOALLOC_TABLE_BYTES that the library holds in a file-scope device array on each GPU
- * until the process ends, and reach it through the arguments of small copy kernels on
- * `stream`.  A call whose tables exceed that area (about 3,400 tensors) fails with AW4_EINVAL.
+ * AW4_NOALLOC_TABLE_BYTES (and the headers of further launches) that the library holds in a
+ * file-scope device array on each GPU until the process ends, and reach it through the arguments
+ * of small copy kernels on `stream`.  A call of more tensors than AW4_NOALLOC_TABLE_BYTES holds
+ * in one table (3,449), however many launches they take, fails with AW4_EINVAL.
  * The first call on a device (of any entry point) copies the codebook tables to it once,
  * synchronously.  Every call on one GPU uses the same area: calls on one stream are ordered,
  * calls that overlap on different streams of one GPU race.

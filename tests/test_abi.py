@@ -422,6 +422,31 @@ def test_noalloc_step_rejects_tables_beyond_its_area():
     assert b"tensor 7: numel 0" in lib.aw4_last_error()
 
 
+@pytest.mark.parametrize("kinds", ["fp32 state", "blocks and fp32 state", "three dtypes"])
+def test_noalloc_step_takes_every_split_of_a_table_that_fits(kinds):
+    """The 3,449 tensors that AW4_NOALLOC_TABLE_BYTES holds in one table are not refused for the headers
+    and the padding of further launches (no kernel of the step runs: its launch is made to fail)."""
+    lib = _lib.library()
+    n = (_lib.NOALLOC_TABLE_BYTES - 64) // (_lib.TENSOR.itemsize + 8)
+    assert n == 3449
+    for count, refused in ((n, False), (n + 1, True)):
+        rows = np.zeros(count, dtype=_lib.TENSOR)
+        rows["param"], rows["grad"], rows["numel"] = 1 << 20, 2 << 20, 100
+        rows["m1"]["values"], rows["m2"]["values"] = 3 << 20, 4 << 20
+        rows["m1"]["rounding"] = rows["m2"]["rounding"] = _lib.ROUND_FP32
+        if kinds == "blocks and fp32 state":  # a block launch that the fp32-state tensors do not join
+            for m in ("m1", "m2"):
+                rows[m]["rounding"][0] = _lib.ROUND_RTN
+                rows[m]["codes"][0], rows[m]["scales"][0] = 5 << 20, 6 << 20
+            rows["numel"][0], rows["flags"][0] = 8192 * 1024, _lib.TENSOR_VEC_ALIGNED
+        elif kinds == "three dtypes":
+            rows["param_dtype"] = rows["grad_dtype"] = np.arange(count) % 3
+        lib.aw4_inject_launch_failure(0)
+        rc = lib.aw4_fused_step_noalloc(rows.ctypes.data, count, None)
+        lib.aw4_inject_launch_failure(-1)
+        assert (rc == _lib.EINVAL) == refused, (kinds, count, lib.aw4_last_error())
+
+
 def test_step_rejects_unknown_dtypes_and_scaled_float64_gradients():
     """Rows are checked before any device work (no GPU needed): a dtype code outside
     AW4_F32/BF16/F16/F64 fails, and so does a float64 gradient with GRAD_SCALE or GRAD_UNSCALE (the
