@@ -737,10 +737,8 @@ struct StagingSlot {
     const void* host_dev = nullptr;  // the device's address of `host`
     void* dev = nullptr;             // device copy the kernels read
     size_t cap = 0;
-    // The norm pass's workgroup counters, behind `dev`, zero outside its launches: the gradients', and the
-    // segment groups'.
-    uint32_t* tickets = nullptr;
-    uint32_t* ticket_groups = nullptr;
+    uint32_t* counters = nullptr;    // the norm pass's (norm_counters), zero outside its launches
+    size_t counter_words = 0;
     hipEvent_t done = nullptr;
     bool pending = false;
 };
@@ -1046,14 +1044,7 @@ int acquire_slot(DeviceState* ds, size_t bytes, StagingSlot** out) {
         void* mapped = nullptr;
         AW4_HIP_CHECK(hipHostGetDevicePointer(&mapped, slot.host, 0));
         slot.host_dev = mapped;
-        // The counters: one per gradient and one more, and those of the segment groups, of a pass that keeps
-        // 8 bytes per gradient and per segment in `dev`.
-        const size_t words = (cap / 8 + 1 + kNormGroupStride - 1) / kNormGroupStride * kNormGroupStride;
-        const std::vector<uint32_t> zero(words + (size_t)norm_group_words((int64_t)(cap / 8)), 0u);
-        AW4_HIP_CHECK(hipMalloc(&slot.dev, cap + zero.size() * sizeof(uint32_t)));
-        slot.tickets = (uint32_t*)((char*)slot.dev + cap);
-        slot.ticket_groups = slot.tickets + words;
-        AW4_HIP_CHECK(hipMemcpy(slot.tickets, zero.data(), zero.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        AW4_HIP_CHECK(hipMalloc(&slot.dev, cap));
         slot.cap = cap;
     }
     // The event only tells the host that the launch which read the slot has finished; no data
@@ -1419,6 +1410,31 @@ int norm_segment_shift(int64_t values) {
 
 int64_t norm_segments(int64_t numel, int shift) { return (numel + ((int64_t)1 << shift) - 1) >> shift; }
 
+__global__ void __launch_bounds__(kStageThreads) zero_words_kernel(uint32_t* dst, int64_t n) {
+    for (int64_t i = (int64_t)blockIdx.x * kStageThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kStageThreads)
+        dst[i] = 0;
+}
+
+// The workgroup counters of a norm pass over `slot` (acquired: its last launch has completed), at least
+// `words` of them.  Only the norm pass allocates them, and a kernel before its launch clears new ones: a
+// synchronous copy of zeros would have the host wait for all work queued so far.
+int norm_counters(StagingSlot& slot, size_t words, hipStream_t s) {
+    if (slot.counter_words >= words) return AW4_OK;
+    slot.counter_words = 0;
+    if (slot.counters) AW4_HIP_CHECK(hipFree(slot.counters));
+    slot.counters = nullptr;
+    size_t cap = 1024;
+    while (cap < words) cap *= 2;
+    void* p = nullptr;
+    AW4_HIP_CHECK(hipMalloc(&p, cap * sizeof(uint32_t)));
+    slot.counters = (uint32_t*)p;
+    const size_t blocks = std::min<size_t>((cap + kStageThreads - 1) / kStageThreads, 1024);
+    hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)blocks), dim3(kStageThreads), 0, s, slot.counters, (int64_t)cap);
+    AW4_HIP_CHECK(hipGetLastError());
+    slot.counter_words = cap;
+    return AW4_OK;
+}
+
 // The norm pass and coefficient of aw4_clip_coefficient (inv_scale null) and
 // aw4_unscale_clip_coefficient.
 int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, const float* inv_scale,
@@ -1462,6 +1478,11 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     StagingSlot* slot = nullptr;
     rc = acquire_slot(ds, bytes, &slot);
     if (rc) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    // one counter per gradient and one more, then the segment groups'
+    const size_t gradient_words = ((size_t)count + 1 + kNormGroupStride - 1) / kNormGroupStride * kNormGroupStride;
+    rc = norm_counters(*slot, gradient_words + (size_t)norm_group_words(segments), s);
+    if (rc) return rc;
     NormInlineArgs args;
     NormHeader* h = (NormHeader*)(in_args ? (void*)args.table : slot->host);
     memset(h, 0, sizeof(*h));
@@ -1481,8 +1502,8 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     h->segment_shift = shift;
     h->partials = (uint64_t)slot->dev + scratch_at;
     h->norm_sq = h->partials + sizeof(double) * (uint64_t)segments;
-    h->tickets = (uint64_t)slot->tickets;
-    h->groups = (uint64_t)slot->ticket_groups;
+    h->tickets = (uint64_t)slot->counters;
+    h->groups = (uint64_t)(slot->counters + gradient_words);
     h->norm_out = (uint64_t)norm_out;
     h->coef_out = (uint64_t)coef_out;
     if (unscale) {
@@ -1490,17 +1511,21 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
         h->nonfinite = h->norm_sq + sizeof(double) * (uint64_t)count;
         h->found_out = (uint64_t)found_out;
     }
-    hipStream_t s = (hipStream_t)stream;
     if (in_args) {
         hipLaunchKernelGGL(norm_kernel_inline, dim3((unsigned)segments), dim3(kNormThreads), 0, s, args);
     } else {
         rc = upload_slot(*slot, table, s);
-        if (rc) return rc;
-        hipLaunchKernelGGL(norm_kernel, dim3((unsigned)segments), dim3(kNormThreads), 0, s, (const NormHeader*)slot->dev);
+        if (!rc)
+            hipLaunchKernelGGL(norm_kernel, dim3((unsigned)segments), dim3(kNormThreads), 0, s, (const NormHeader*)slot->dev);
     }
-    AW4_HIP_CHECK(hipGetLastError());
-    AW4_HIP_CHECK(hipEventRecord(slot->done, s));
-    slot->pending = true;
+    const hipError_t launched = rc ? hipSuccess : hipGetLastError();
+    // the slot is in use by whatever was enqueued; if that cannot be waited for, its counters are not used again
+    const hipError_t err = hipEventRecord(slot->done, s);
+    slot->pending = err == hipSuccess;
+    if (err != hipSuccess) slot->counter_words = 0;
+    if (rc) return rc;
+    AW4_HIP_CHECK(launched);
+    AW4_HIP_CHECK(err);
     return AW4_OK;
 }
 
