@@ -62,6 +62,13 @@ constexpr int kNormGroup = 32, kNormGroupStride = 32;
 __host__ __device__ constexpr int64_t norm_group_words(int64_t segments) {
     return 2 * kNormGroupStride * (segments / kNormGroup + 1);
 }
+// Finished gradients likewise, from kNormManyGradients on: a ticket for each aligned run of kNormGroup of
+// them, behind the segments' runs.  (From 64 on measured the same at 150 and 200 gradients, whose one counter
+// is no longer than the further level's latency.)
+constexpr int kNormManyGradients = 256;
+__host__ __device__ constexpr int64_t norm_many_words(int64_t gradients) {
+    return gradients < kNormManyGradients ? 0 : kNormGroupStride * (gradients / kNormGroup + 1);
+}
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
@@ -148,6 +155,7 @@ __device__ __forceinline__ uint32_t draw_ticket(gptr<uint32_t> p) {
 // Draws for one finished segment of gradient t (segments start .. end - 1); whether it was the gradient's last.
 __device__ __forceinline__ bool norm_last_of_gradient(const NormHeader* hdr, int t, int seg, int start, int end) {
     uint32_t drawers = (uint32_t)(end - start);
+    if (drawers == 1u) return true;
     if (end - start > kNormGroup) {
         const int run = seg / kNormGroup, run0 = run * kNormGroup;
         const gptr<uint32_t> group =
@@ -160,6 +168,20 @@ __device__ __forceinline__ bool norm_last_of_gradient(const NormHeader* hdr, int
     return draw_ticket(gaddr<uint32_t>(hdr->tickets) + t) == drawers - 1u;
 }
 
+// Draws for finished gradient t; whether it was the launch's last.
+__device__ __forceinline__ bool norm_last_of_all(const NormHeader* hdr, int t, int count) {
+    uint32_t drawers = (uint32_t)count;
+    if (count >= kNormManyGradients) {
+        const int run = t / kNormGroup, run0 = run * kNormGroup;
+        const gptr<uint32_t> group =
+            gaddr<uint32_t>(hdr->groups) + norm_group_words(hdr->total_segments) + kNormGroupStride * (int64_t)run;
+        if (draw_ticket(group) != (uint32_t)(min(count, run0 + kNormGroup) - run0) - 1u) return false;
+        agent_store(group, 0u);
+        drawers = (uint32_t)((count - 1) / kNormGroup + 1);
+    }
+    return draw_ticket(gaddr<uint32_t>(hdr->tickets) + count) == drawers - 1u;
+}
+
 // The index of the gradient that holds a segment.
 __device__ __forceinline__ int norm_row_of(const NormRow* rows, int count, int seg) {
     int lo = 0, hi = count - 1;
@@ -168,6 +190,11 @@ __device__ __forceinline__ int norm_row_of(const NormRow* rows, int count, int s
         if (rows[mid].seg_start <= seg) lo = mid; else hi = mid - 1;
     }
     return lo;
+}
+
+__device__ __forceinline__ double norm_sq_of(double s, int dtype) {
+    const float norm_t = round_to_dtype((float)__builtin_sqrt(s), dtype);
+    return (double)norm_t * (double)norm_t;  // exact
 }
 
 // norm_t^2 of one gradient from its segments' sums (lanes stride over them): wave 0 of its last workgroup.
@@ -183,9 +210,7 @@ __device__ __forceinline__ double norm_tensor_sq(const NormHeader* hdr, int firs
         for (int i = 0; i < 8; ++i) s += v[i];
     }
     for (; k < end; k += 64) s += agent_load(partials + k);
-    s = wave_sum_f64(s);
-    const float norm_t = round_to_dtype((float)__builtin_sqrt(s), dtype);
-    return (double)norm_t * (double)norm_t;  // exact
+    return norm_sq_of(wave_sum_f64(s), dtype);
 }
 
 // The total norm and the coefficient, by the whole of the launch's last workgroup: thread i adds
@@ -196,8 +221,17 @@ __device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_
     const gptr<uint32_t> tickets = gaddr<uint32_t>(hdr->tickets);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double sq = 0.0;
-    for (int t = threadIdx.x; t < count; t += kNormThreads) sq += agent_load(norm_sq + t);
-    for (int t = threadIdx.x; t <= count; t += kNormThreads) tickets[t] = 0;  // every workgroup has drawn its own
+    int at = threadIdx.x;
+    for (; at + 7 * kNormThreads < count; at += 8 * kNormThreads) {
+        double v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = agent_load(norm_sq + at + kNormThreads * i);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sq += v[i];
+    }
+    for (; at < count; at += kNormThreads) sq += agent_load(norm_sq + at);
+    // every workgroup has drawn its own: plain stores, complete for the next launch at this one's end
+    for (int t = threadIdx.x; t <= count; t += kNormThreads) tickets[t] = 0;
     sq = wave_sum_f64(sq);
     uint32_t bad = 0;
     if (hdr->unscale) {
@@ -249,6 +283,9 @@ __device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_
 // 135 -> 127 us, 9 MB of bf16 gradients in seven tensors 82 -> 73 us.
 // With tickets in two levels and the partials loaded eight at a time: one 4096^2 fp32 gradient's pass 40 us
 // (1.7 TB/s) -> 16, clip and step 89.8 -> 65.9 us; two bf16 ones 124.4 -> 104.2 us.
+// Many gradients, host and pass (fp32, of 1,000 values): drawing from one counter each 1,000 gradients took
+// 24.7 us, 5,000 78.0 and 20,000 275; in runs, and without tickets for a gradient's only segment, 15.1, 28.6
+// and 83.9.
 __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
     const NormRow* rows = (const NormRow*)(hdr + 1);
     const int count = hdr->count;
@@ -277,12 +314,12 @@ __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
     __shared__ double wave_acc[kNormThreads / 64];
     __shared__ uint32_t wave_bad_any[kNormThreads / 64];
     __shared__ uint32_t last_of_gradient, last_of_all;  // this workgroup drew the last ticket
+    const bool whole = end - T.seg_start == 1;          // the gradient's only segment
     if ((threadIdx.x & 63) == 0) {
         wave_acc[threadIdx.x >> 6] = acc;
         wave_bad_any[threadIdx.x >> 6] = wave_bad ? 1u : 0u;
     }
     __syncthreads();
-    const gptr<uint32_t> tickets = gaddr<uint32_t>(hdr->tickets);
     if (threadIdx.x == 0) {
         double s = wave_acc[0];
         uint32_t b = wave_bad_any[0];
@@ -291,17 +328,19 @@ __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
             s += wave_acc[w];
             b |= wave_bad_any[w];
         }
-        agent_store(gaddr<double>(hdr->partials) + seg, s);
+        if (whole) wave_acc[0] = s;
+        else agent_store(gaddr<double>(hdr->partials) + seg, s);
         if (hdr->unscale) agent_store(gaddr<uint32_t>(hdr->nonfinite) + seg, b);
         last_of_gradient = norm_last_of_gradient(hdr, t, seg, T.seg_start, end) ? 1u : 0u;
     }
     __syncthreads();
     if (!last_of_gradient) return;
     if (threadIdx.x < 64) {
-        const double norm_sq = norm_tensor_sq(hdr, T.seg_start, end, dtype);
+        const double norm_sq =
+            whole ? norm_sq_of(wave_acc[0], dtype) : norm_tensor_sq(hdr, T.seg_start, end, dtype);
         if (threadIdx.x == 0) {
             agent_store(gaddr<double>(hdr->norm_sq) + t, norm_sq);
-            last_of_all = draw_ticket(tickets + count) == (uint32_t)count - 1u ? 1u : 0u;
+            last_of_all = norm_last_of_all(hdr, t, count) ? 1u : 0u;
         }
     }
     __syncthreads();

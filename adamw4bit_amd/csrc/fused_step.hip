@@ -1479,9 +1479,9 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     rc = acquire_slot(ds, bytes, &slot);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    // one counter per gradient and one more, then the segment groups'
+    // one counter per gradient and one more, then those of the runs of segments and of gradients
     const size_t gradient_words = ((size_t)count + 1 + kNormGroupStride - 1) / kNormGroupStride * kNormGroupStride;
-    rc = norm_counters(*slot, gradient_words + (size_t)norm_group_words(segments), s);
+    rc = norm_counters(*slot, gradient_words + (size_t)(norm_group_words(segments) + norm_many_words(count)), s);
     if (rc) return rc;
     NormInlineArgs args;
     NormHeader* h = (NormHeader*)(in_args ? (void*)args.table : slot->host);
