@@ -104,16 +104,18 @@ template <int G, bool kUnscale>
 __device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t e1, bool vec, float u,
                                               bool& bad) {
     // Full groups of 4 values: thread i takes groups i, i + 256, ... (8 loads in flight per
-    // thread: 4 KB per workgroup per load instruction).
+    // thread: 4 KB per workgroup per load instruction; 4 where fp16 values are unscaled, which with 8 took the
+    // kernel from 44 to 69 VGPRs and an eighth workgroup from each CU).
+    constexpr int kLoads = kUnscale && G == D_F16 ? 4 : 8;
     double acc = 0.0;
     const int64_t groups = (e1 - e0) >> 2;
     int64_t k = threadIdx.x;
-    for (; k + 7 * kNormThreads < groups; k += 8 * kNormThreads) {
-        double s[8];
+    for (; k + (kLoads - 1) * kNormThreads < groups; k += kLoads * kNormThreads) {
+        double s[kLoads];
 #pragma unroll
-        for (int v = 0; v < 8; ++v) s[v] = sq4<G, kUnscale>(grad, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
+        for (int v = 0; v < kLoads; ++v) s[v] = sq4<G, kUnscale>(grad, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
 #pragma unroll
-        for (int v = 0; v < 8; ++v) acc += s[v];
+        for (int v = 0; v < kLoads; ++v) acc += s[v];
     }
     for (; k < groups; k += kNormThreads) acc += sq4<G, kUnscale>(grad, e0 + 4 * k, vec, u, bad);
     // the tail of the tensor (fewer than 4 values)
