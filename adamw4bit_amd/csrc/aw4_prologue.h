@@ -44,8 +44,9 @@ struct NormHeader {
     int32_t segment_shift;
     uint64_t partials;     // device address, double[total_segments]
     uint64_t norm_sq;      // device address, double[count]: norm_t^2 of each gradient
-    uint64_t tickets;      // device address, uint32[count + 1], zero before and after the launch
-    uint64_t groups;       // device address, the segment groups' tickets (norm_group_words), likewise
+    uint64_t tickets;      // device address, the gradients' tickets and the launch's (norm_ticket_words), zero
+                           // before and after the launch
+    uint64_t groups;       // device address, the segment groups' (norm_group_words), likewise
     uint64_t norm_out;     // device address, float
     uint64_t coef_out;     // device address, float
     uint64_t inv_scale;    // device address, float u (unscale)
@@ -54,20 +55,23 @@ struct NormHeader {
 };
 // followed by NormRow rows[count]
 
-// A gradient of more than kNormGroup segments counts them in two levels, a ticket for each aligned run of
-// kNormGroup segments (the gradient's part of it) and the gradient's for its runs: atomics on one address
-// follow one another at about 14 ns, 2,048 segments of one gradient for 28 us.  A run holds parts of at most
-// two such gradients, one that starts in it and one before: two tickets each, each in a cache line of its own.
-constexpr int kNormGroup = 32, kNormGroupStride = 32;
+// Every ticket is in a cache line of its own, and whoever draws a ticket's last number clears it: atomics on one
+// line follow one another at about 14 ns, and a launch's workgroups finish together (2 GB in 64 fp32 gradients of
+// 32 segments: 357 us with their tickets in two lines).  For the same reason a gradient of more than kNormGroup
+// segments counts them in two levels, a ticket for each aligned run of kNormGroup segments (the gradient's part
+// of it) and the gradient's for its runs.  A run holds parts of at most two such gradients, one that starts in
+// it and one before: two tickets each.
+constexpr int kNormGroup = 32, kNormTicketStride = 32;
+__host__ __device__ constexpr int64_t norm_ticket_words(int64_t gradients) { return kNormTicketStride * (gradients + 1); }
 __host__ __device__ constexpr int64_t norm_group_words(int64_t segments) {
-    return 2 * kNormGroupStride * (segments / kNormGroup + 1);
+    return 2 * kNormTicketStride * (segments / kNormGroup + 1);
 }
 // Finished gradients likewise, from kNormManyGradients on: a ticket for each aligned run of kNormGroup of
 // them, behind the segments' runs.  (From 64 on measured the same at 150 and 200 gradients, whose one counter
 // is no longer than the further level's latency.)
 constexpr int kNormManyGradients = 256;
 __host__ __device__ constexpr int64_t norm_many_words(int64_t gradients) {
-    return gradients < kNormManyGradients ? 0 : kNormGroupStride * (gradients / kNormGroup + 1);
+    return gradients < kNormManyGradients ? 0 : kNormTicketStride * (gradients / kNormGroup + 1);
 }
 
 __device__ __forceinline__ double wave_sum_f64(double v) {
@@ -132,9 +136,17 @@ __device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t
     return acc;
 }
 
+template <bool kUnscale>
+__device__ __forceinline__ double segment_sum_any(uint64_t grad, int dtype, int64_t e0, int64_t e1, bool vec, float u,
+                                                  bool& bad) {
+    if (dtype == D_F32) return segment_sum<D_F32, kUnscale>(grad, e0, e1, vec, u, bad);
+    if (dtype == D_BF16) return segment_sum<D_BF16, kUnscale>(grad, e0, e1, vec, u, bad);
+    return segment_sum<D_F16, kUnscale>(grad, e0, e1, vec, u, bad);
+}
+
 // What one workgroup leaves for another goes through device-scope atomic accesses only (the XCDs' L2
 // caches are not coherent for plain ones within a launch): a store written through, complete when
-// draw_ticket's wait returns, then the ticket, and loads past the caches by whoever drew the last one.
+// draw_last's wait returns, then the ticket, and loads past the caches by whoever drew the last one.
 // A release and an acquire in their place would also write back and invalidate an L2 per workgroup, for
 // plain stores that none of them reads: 195 us a pass more for GPT-2-small, after a step's dirty lines.
 template <class T>
@@ -146,28 +158,29 @@ __device__ __forceinline__ void agent_store(gptr<T> p, T v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ uint32_t draw_ticket(gptr<uint32_t> p) {
+// Whether this was the last of `drawers` draws of a ticket, which it then leaves cleared.
+__device__ __forceinline__ bool draw_last(gptr<uint32_t> p, uint32_t drawers) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keeps the order in the compiler
     __builtin_amdgcn_s_waitcnt(0x0F70);                     // vmcnt(0): this thread's stores are complete
     const uint32_t drawn = __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    return drawn;
+    if (drawn != drawers - 1u) return false;
+    agent_store(p, 0u);
+    return true;
 }
 
 // Draws for one finished segment of gradient t (segments start .. end - 1); whether it was the gradient's last.
 __device__ __forceinline__ bool norm_last_of_gradient(const NormHeader* hdr, int t, int seg, int start, int end) {
     uint32_t drawers = (uint32_t)(end - start);
     if (drawers == 1u) return true;
-    if (end - start > kNormGroup) {
+    if (drawers > (uint32_t)kNormGroup) {
         const int run = seg / kNormGroup, run0 = run * kNormGroup;
         const gptr<uint32_t> group =
-            gaddr<uint32_t>(hdr->groups) + kNormGroupStride * (2 * (int64_t)run + (start > run0 ? 1 : 0));
-        const int segments = min(end, run0 + kNormGroup) - max(start, run0);
-        if (draw_ticket(group) != (uint32_t)segments - 1u) return false;
-        agent_store(group, 0u);  // all of its segments have drawn
+            gaddr<uint32_t>(hdr->groups) + kNormTicketStride * (2 * (int64_t)run + (start > run0 ? 1 : 0));
+        if (!draw_last(group, (uint32_t)(min(end, run0 + kNormGroup) - max(start, run0)))) return false;
         drawers = (uint32_t)((end - 1) / kNormGroup - start / kNormGroup + 1);
     }
-    return draw_ticket(gaddr<uint32_t>(hdr->tickets) + t) == drawers - 1u;
+    return draw_last(gaddr<uint32_t>(hdr->tickets) + kNormTicketStride * (int64_t)t, drawers);
 }
 
 // Draws for finished gradient t; whether it was the launch's last.
@@ -176,12 +189,11 @@ __device__ __forceinline__ bool norm_last_of_all(const NormHeader* hdr, int t, i
     if (count >= kNormManyGradients) {
         const int run = t / kNormGroup, run0 = run * kNormGroup;
         const gptr<uint32_t> group =
-            gaddr<uint32_t>(hdr->groups) + norm_group_words(hdr->total_segments) + kNormGroupStride * (int64_t)run;
-        if (draw_ticket(group) != (uint32_t)(min(count, run0 + kNormGroup) - run0) - 1u) return false;
-        agent_store(group, 0u);
+            gaddr<uint32_t>(hdr->groups) + norm_group_words(hdr->total_segments) + kNormTicketStride * (int64_t)run;
+        if (!draw_last(group, (uint32_t)(min(count, run0 + kNormGroup) - run0))) return false;
         drawers = (uint32_t)((count - 1) / kNormGroup + 1);
     }
-    return draw_ticket(gaddr<uint32_t>(hdr->tickets) + count) == drawers - 1u;
+    return draw_last(gaddr<uint32_t>(hdr->tickets) + kNormTicketStride * (int64_t)count, drawers);
 }
 
 // The index of the gradient that holds a segment.
@@ -220,7 +232,6 @@ __device__ __forceinline__ double norm_tensor_sq(const NormHeader* hdr, int firs
 __device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_sq, uint32_t* wave_bad_any) {
     const int count = hdr->count;
     const gptr<double> norm_sq = gaddr<double>(hdr->norm_sq);
-    const gptr<uint32_t> tickets = gaddr<uint32_t>(hdr->tickets);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double sq = 0.0;
     int at = threadIdx.x;
@@ -232,8 +243,6 @@ __device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_
         for (int i = 0; i < 8; ++i) sq += v[i];
     }
     for (; at < count; at += kNormThreads) sq += agent_load(norm_sq + at);
-    // every workgroup has drawn its own: plain stores, complete for the next launch at this one's end
-    for (int t = threadIdx.x; t <= count; t += kNormThreads) tickets[t] = 0;
     sq = wave_sum_f64(sq);
     uint32_t bad = 0;
     if (hdr->unscale) {
@@ -286,8 +295,9 @@ __device__ __forceinline__ void norm_finish(const NormHeader* hdr, double* wave_
 // With tickets in two levels and the partials loaded eight at a time: one 4096^2 fp32 gradient's pass 40 us
 // (1.7 TB/s) -> 16, clip and step 89.8 -> 65.9 us; two bf16 ones 124.4 -> 104.2 us.
 // Many gradients, host and pass (fp32, of 1,000 values): drawing from one counter each 1,000 gradients took
-// 24.7 us, 5,000 78.0 and 20,000 275; in runs, and without tickets for a gradient's only segment, 15.1, 28.6
-// and 83.9.
+// 24.7 us, 5,000 78.0 and 20,000 275; in runs, and without tickets for a gradient's only segment, 14.7, 27.5
+// and 79.  With every ticket in a line of its own: 512 MB of bf16 gradients in 64 tensors 178 -> 165 us, 2 GB of
+// fp32 ones 357 -> 311 (both read past the caches).
 __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
     const NormRow* rows = (const NormRow*)(hdr + 1);
     const int count = hdr->count;
@@ -303,13 +313,9 @@ __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
     bool bad = false;
     if (hdr->unscale) {
         const float u = *gaddr<const float>(hdr->inv_scale);
-        if (dtype == D_F32) acc = segment_sum<D_F32, true>(T.grad, e0, e1, vec, u, bad);
-        else if (dtype == D_BF16) acc = segment_sum<D_BF16, true>(T.grad, e0, e1, vec, u, bad);
-        else acc = segment_sum<D_F16, true>(T.grad, e0, e1, vec, u, bad);
+        acc = segment_sum_any<true>(T.grad, dtype, e0, e1, vec, u, bad);
     } else {
-        if (dtype == D_F32) acc = segment_sum<D_F32, false>(T.grad, e0, e1, vec, 1.0f, bad);
-        else if (dtype == D_BF16) acc = segment_sum<D_BF16, false>(T.grad, e0, e1, vec, 1.0f, bad);
-        else acc = segment_sum<D_F16, false>(T.grad, e0, e1, vec, 1.0f, bad);
+        acc = segment_sum_any<false>(T.grad, dtype, e0, e1, vec, 1.0f, bad);
     }
     acc = wave_sum_f64(acc);
     const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;

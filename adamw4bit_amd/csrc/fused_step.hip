@@ -1479,9 +1479,8 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     rc = acquire_slot(ds, bytes, &slot);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    // one counter per gradient and one more, then those of the runs of segments and of gradients
-    const size_t gradient_words = ((size_t)count + 1 + kNormGroupStride - 1) / kNormGroupStride * kNormGroupStride;
-    rc = norm_counters(*slot, gradient_words + (size_t)(norm_group_words(segments) + norm_many_words(count)), s);
+    const int64_t ticket_words = norm_ticket_words(count);
+    rc = norm_counters(*slot, (size_t)(ticket_words + norm_group_words(segments) + norm_many_words(count)), s);
     if (rc) return rc;
     NormInlineArgs args;
     NormHeader* h = (NormHeader*)(in_args ? (void*)args.table : slot->host);
@@ -1503,7 +1502,7 @@ int norm_prologue(const char* what, const aw4_tensor* tensors, int32_t count, co
     h->partials = (uint64_t)slot->dev + scratch_at;
     h->norm_sq = h->partials + sizeof(double) * (uint64_t)segments;
     h->tickets = (uint64_t)slot->counters;
-    h->groups = (uint64_t)(slot->counters + gradient_words);
+    h->groups = (uint64_t)(slot->counters + ticket_words);
     h->norm_out = (uint64_t)norm_out;
     h->coef_out = (uint64_t)coef_out;
     if (unscale) {
