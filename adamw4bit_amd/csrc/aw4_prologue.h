@@ -31,9 +31,10 @@ struct NormRow {
     uint64_t grad;      // device address
     int64_t numel;
     int32_t seg_start;  // first of its segments
-    int32_t dtype;      // AW4_* of the gradient, with kNormVec where 4-value vector access is allowed
+    int32_t dtype;      // AW4_* of the gradient, with kNormVec where 4-value vector access is allowed and
+                        // kNormKeep where the loads go through the caches
 };
-constexpr int kNormVec = 0x100;
+constexpr int kNormVec = 0x100, kNormKeep = 0x200;
 
 struct NormHeader {
     int32_t count;
@@ -92,11 +93,11 @@ __device__ __forceinline__ double sq1(float f, float u, bool& bad) {
 }
 
 // Sum of squares of 4 consecutive gradient values starting at element e (all in range).
-template <int G, bool kUnscale>
+template <int G, bool kUnscale, bool kKeep>
 __device__ __forceinline__ double sq4(uint64_t grad, int64_t e, bool vec, float u, bool& bad) {
     uint32_t w[4];
     float f[4];
-    load_words<G, true>(grad, e, vec, w);
+    load_words<G, kKeep>(grad, e, vec, w);
     words_to_f32<G>(w, f);
     double s = 0.0;
 #pragma unroll
@@ -104,7 +105,7 @@ __device__ __forceinline__ double sq4(uint64_t grad, int64_t e, bool vec, float 
     return s;
 }
 
-template <int G, bool kUnscale>
+template <int G, bool kUnscale, bool kKeep>
 __device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t e1, bool vec, float u,
                                               bool& bad) {
     // Full groups of 4 values: thread i takes groups i, i + 256, ... (8 loads in flight per
@@ -117,11 +118,11 @@ __device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t
     for (; k + (kLoads - 1) * kNormThreads < groups; k += kLoads * kNormThreads) {
         double s[kLoads];
 #pragma unroll
-        for (int v = 0; v < kLoads; ++v) s[v] = sq4<G, kUnscale>(grad, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
+        for (int v = 0; v < kLoads; ++v) s[v] = sq4<G, kUnscale, kKeep>(grad, e0 + 4 * (k + v * kNormThreads), vec, u, bad);
 #pragma unroll
         for (int v = 0; v < kLoads; ++v) acc += s[v];
     }
-    for (; k < groups; k += kNormThreads) acc += sq4<G, kUnscale>(grad, e0 + 4 * k, vec, u, bad);
+    for (; k < groups; k += kNormThreads) acc += sq4<G, kUnscale, kKeep>(grad, e0 + 4 * k, vec, u, bad);
     // the tail of the tensor (fewer than 4 values)
     const int64_t tail = e0 + 4 * groups;
     if ((int64_t)threadIdx.x < e1 - tail) {
@@ -136,12 +137,12 @@ __device__ __forceinline__ double segment_sum(uint64_t grad, int64_t e0, int64_t
     return acc;
 }
 
-template <bool kUnscale>
+template <bool kUnscale, bool kKeep>
 __device__ __forceinline__ double segment_sum_any(uint64_t grad, int dtype, int64_t e0, int64_t e1, bool vec, float u,
                                                   bool& bad) {
-    if (dtype == D_F32) return segment_sum<D_F32, kUnscale>(grad, e0, e1, vec, u, bad);
-    if (dtype == D_BF16) return segment_sum<D_BF16, kUnscale>(grad, e0, e1, vec, u, bad);
-    return segment_sum<D_F16, kUnscale>(grad, e0, e1, vec, u, bad);
+    if (dtype == D_F32) return segment_sum<D_F32, kUnscale, kKeep>(grad, e0, e1, vec, u, bad);
+    if (dtype == D_BF16) return segment_sum<D_BF16, kUnscale, kKeep>(grad, e0, e1, vec, u, bad);
+    return segment_sum<D_F16, kUnscale, kKeep>(grad, e0, e1, vec, u, bad);
 }
 
 // What one workgroup leaves for another goes through device-scope atomic accesses only (the XCDs' L2
@@ -311,11 +312,14 @@ __device__ __forceinline__ void norm_body(const NormHeader* hdr) {
     const bool vec = (T.dtype & kNormVec) != 0;
     double acc;
     bool bad = false;
+    const bool keep = (T.dtype & kNormKeep) != 0;
     if (hdr->unscale) {
         const float u = *gaddr<const float>(hdr->inv_scale);
-        acc = segment_sum_any<true>(T.grad, dtype, e0, e1, vec, u, bad);
+        acc = keep ? segment_sum_any<true, true>(T.grad, dtype, e0, e1, vec, u, bad)
+                   : segment_sum_any<true, false>(T.grad, dtype, e0, e1, vec, u, bad);
     } else {
-        acc = segment_sum_any<false>(T.grad, dtype, e0, e1, vec, 1.0f, bad);
+        acc = keep ? segment_sum_any<false, true>(T.grad, dtype, e0, e1, vec, 1.0f, bad)
+                   : segment_sum_any<false, false>(T.grad, dtype, e0, e1, vec, 1.0f, bad);
     }
     acc = wave_sum_f64(acc);
     const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;

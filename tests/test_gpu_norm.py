@@ -80,6 +80,26 @@ def test_many_gradients_do_not_draw_one_after_another():
     assert min(times) < 8e-3 * count, times
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_loads_through_and_past_the_caches(dtype):
+    """160 * 2^20 values, the most that are read through the caches, and one more; the gradients one value off
+    their alignment too.  Against the sums of 2^20 values each, added in float64."""
+    most = 160 << 20
+    gen = torch.Generator(device=H.DEVICE).manual_seed(9)
+    flat = torch.empty(most + 8, device=H.DEVICE, dtype=dtype).normal_(generator=gen)
+    for sizes, shift in (((most - 3, 3), 0), ((most - 3, 4), 0), ((most, 1), 1)):
+        a = flat[shift:shift + sizes[0]]
+        grads = [a, flat[most + 4 - sizes[1]:most + 4]]
+        sq = math.fsum(float(c.double().square().sum()) for c in a.split(1 << 20))
+        per = [torch.tensor(math.sqrt(sq), dtype=torch.float64).float().to(dtype).double(),
+               grads[1].double().square().sum().sqrt().float().to(dtype).double().cpu()]
+        want = float(torch.stack(per).square().sum().sqrt().float().to(dtype))
+        for _ in range(2):
+            # the order of the float64 sums differs: a relative 2^-40 at most, one rounding of the norm where it is a tie
+            got = norm_pass(grads)[0]
+            assert abs(got - want) <= H.ULP16.get(dtype, 2.0 ** -23) * want, (sizes, got, want)
+
+
 @pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
 @pytest.mark.parametrize("where", ["first segment", "inside", "last segment of a cut gradient", "second gradient"])
 def test_unscaling_finds_values_that_are_not_finite(where, bad):
