@@ -106,7 +106,7 @@ struct LdsSlots {
     PairEntry pairs[2][kPairs];
     SsrEntry ssr[kSsr ? 2 : 1][kPairs];
     float2 dec[2][256];
-    LinEntry lin[2][kLinSlots];
+    __align__(16) LinEntry lin[2][kLinSlots];
     WaveScratch scratch[kWavesPerGroup];
     f32x4 m2_stage[kUpd ? kWavesPerGroup * 4 * 64 : 1];  // second moments of a tile (update-SR kernels)
 
@@ -117,22 +117,44 @@ struct LdsSlots {
                             at + ((uint32_t)h->lin_zero[which] << 3) - (f2u(magic) << 3)};
     }
     __device__ f32x4* wave_m2_stage(int wslot) { return kUpd ? &m2_stage[wslot * 4 * 64] : nullptr; }
+    // Every load is issued before the first store to LDS, from addresses that depend on the header alone
+    // (a lookup table is copied whole, whatever its count; a moment without codes copies codebook 0's
+    // tables, which nothing reads): loops over the tables, with a lookup table's count read first, waited
+    // for memory six times in a row at the start of every workgroup.  One fp32 tensor of 2048 x 4096, us so and
+    // with loops: ZIP-SR 26.2 / 28.1, read back after its encode 41.5 / 43.9.
     __device__ void load(const Tables* g, const StepHeader* h) {
-        const int cbs[2] = {h->cb1, h->cb2}, luts[2] = {h->lut1, h->lut2};
+        const int i = threadIdx.x;
+        const int i16 = min(i, 15), ip = min(i, kPairs - 1);
+        float cb_v[2];
+        u32x4 usr_v[2], pair_v[2], ssr_v[2], lin_v[2], lin_last[2];
+        u32x2 dec_v[2];
+#pragma unroll
         for (int w = 0; w < 2; ++w) {
-            if (cbs[w] < 0) continue;
-            for (int i = threadIdx.x; i < 16; i += kThreads) cb[w][i] = g->codebook[cbs[w]][i];
-            for (int i = threadIdx.x; i < kPairs; i += kThreads) usr[w][i] = g->usr[cbs[w]][i];
-            for (int i = threadIdx.x; i < kPairs; i += kThreads) pairs[w][i] = g->pairs[cbs[w]][i];
-            if (kSsr)
-                for (int i = threadIdx.x; i < kPairs; i += kThreads) ssr[w][i] = g->ssr[cbs[w]][i];
-            for (int i = threadIdx.x; i < 256; i += kThreads) dec[w][i] = g->dec[cbs[w]][i];
-            const LinTable& lt = lin_tables(g)[luts[w]];
-            const int n = lt.count;
-            for (int i = threadIdx.x; i < n; i += kThreads) lin[w][i] = lt.e[i];
+            const int c = max(w ? h->cb2 : h->cb1, 0), l = max(w ? h->lut2 : h->lut1, 0);
+            cb_v[w] = g->codebook[c][i16];
+            usr_v[w] = *(const u32x4*)&g->usr[c][ip];
+            pair_v[w] = *(const u32x4*)&g->pairs[c][ip];
+            if (kSsr) ssr_v[w] = *(const u32x4*)&g->ssr[c][ip];
+            dec_v[w] = *(const u32x2*)&g->dec[c][i];
+            const u32x4* e = (const u32x4*)lin_tables(g)[l].e;
+            lin_v[w] = e[i];
+            lin_last[w] = e[kThreads];
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            if (i < 16) cb[w][i] = cb_v[w];
+            if (i < kPairs) {
+                *(u32x4*)&usr[w][i] = usr_v[w];
+                *(u32x4*)&pairs[w][i] = pair_v[w];
+                if (kSsr) *(u32x4*)&ssr[w][i] = ssr_v[w];
+            }
+            *(u32x2*)&dec[w][i] = dec_v[w];
+            *(u32x4*)&lin[w][2 * i] = lin_v[w];
+            if (i == 0) *(u32x4*)&lin[w][2 * kThreads] = lin_last[w];
         }
         __syncthreads();
     }
+    static_assert(kThreads == 256 && kLinSlots == 2 * kThreads + 2, "two lookup entries per thread, and two more");
 };
 
 // Generic kernels: every table.
