@@ -918,10 +918,17 @@ struct LaunchGroup {
 //     24.6 / 30.2; 2048 x 4096 (32) 37.9 / 32.3 and 41.7 / 32.2; 4096^2 (64) 53.3 / 54.5 and
 //     67.9 / 48.8 (a wave of consecutive tiles takes several of them); 14336 x 4096 157.6 / 158.7 and
 //     144.8 / 133.2;
-//   4096^2 and 16 tiles: 64.1 / 53.9 and 78.2 / 48.7.
-constexpr int64_t kValuesLaunchTiles = 1024;  // own launch from this many fp32-state tiles on
-constexpr int64_t kValuesBlockTiles = 8192;   // beside this many block tiles (32 per CU): own launch
-constexpr int64_t kValuesFewTiles = 16;       // ... unless they are fewer than this and in grid order
+//   4096^2 and 16 tiles: 64.1 / 53.9 and 78.2 / 48.7;
+//   1 and 2 tiles beside a large launch, where a wave of consecutive tiles meets two at most: 2048 x 4096 bf16
+//     25.9 / 32.0 and 33.9 / 32.2 (3 and 4: 36.7 / 33.6 and later), 4096^2 40.7 / 47.7 and 46.1 / 47.8,
+//     14336 x 4096 124.2 / 130.1 and 123.1 / 128.9; not so beside the generic kernel, whose one tile takes
+//     longer than a launch: sdyn4_sr / dyn4_sr fp32 2048 x 4096 75.6 / 67.1;
+//   the code-storing lookahead kernels, slower per block tile, hide more of them: fp32 2048 x 4096 and 8 tiles
+//     50.4 / 55.4, bf16 51.0 / 56.0; 16 tiles bf16 4096^2 93.4 / 90.8.
+constexpr int64_t kValuesLaunchTiles = 1024;   // own launch from this many fp32-state tiles on
+constexpr int64_t kValuesBlockTiles = 8192;    // beside this many block tiles (32 per CU): own launch
+constexpr int64_t kValuesFewTiles = 16;        // ... unless they are fewer than this, in grid order or lookahead
+constexpr int64_t kValuesFewConsecutive = 3;   // ... or than this, where waves take consecutive tiles
 
 bool values_variant(const KernelVariant& kv) { return kv.m1 == kFp32 && kv.m2 == kFp32; }
 
@@ -949,8 +956,9 @@ void plan_values(const aw4_tensor* ts, const std::vector<int>& values, std::vect
         if (g && own >= 0) {
             const KernelVariant& kv = kVariants[g->variant];
             const int64_t tiles = tiles_of(ts, of);
-            const bool large = tiles_of(ts, g->members) >= kValuesBlockTiles &&
-                               (tiles >= kValuesFewTiles || !tile_order_grid(kv.m1, kv.m2, kv.dtype));
+            const bool hidden = tile_order_grid(kv.m1, kv.m2, kv.dtype) || kind_of(kv.m2) == K_LA;
+            const int64_t few = g == &generic ? 1 : hidden ? kValuesFewTiles : kValuesFewConsecutive;
+            const bool large = tiles_of(ts, g->members) >= kValuesBlockTiles && tiles >= few;
             if (tiles >= kValuesLaunchTiles || large) g = nullptr;
         }
         if (!g) {

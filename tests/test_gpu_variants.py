@@ -162,3 +162,35 @@ def test_16bit_research_kernels_match_oracle(m2, dtype):
                                         quant_rng_seed=3, optimized=True)
     out = run_pair(make, SHAPES, dtype, 3, seed=3, zero_block_frac=0.02, grad_fn=fp16_safe)
     compare_pair(*out, f"{dtype} nf4/{m2}", steps=3)
+
+
+def launches(params, opt):
+    """How many kernels a step of `opt` launches: the launch after the k-th is made to fail."""
+    lib = _lib.library()
+    for k in range(1, 8):
+        for p in params:
+            p.grad = torch.zeros_like(p)
+        lib.aw4_inject_launch_failure(k)
+        try:
+            opt.step()
+            return k
+        except _lib.HipLaunchIncomplete:
+            opt._inconsistent = None  # the test's own failure; the state is thrown away
+        finally:
+            lib.aw4_inject_launch_failure(-1)
+    raise AssertionError("more launches than the test tries")
+
+
+@pytest.mark.parametrize("dtype,m2,tiles,expect", [
+    (torch.float32, "dyn4_sr", 1, 2),  # the generic kernel, whose fp32-state tile takes longer than a launch
+    (torch.bfloat16, "dyn4_upd_sr_fp32read", 1, 1), (torch.bfloat16, "dyn4_upd_sr_fp32read", 2, 1),
+    (torch.bfloat16, "dyn4_upd_sr_fp32read", 3, 2), (torch.float16, "dyn4_upd_sr_fp32read", 2, 1),
+    (torch.float32, "dyn4_upd_sr", 2, 1), (torch.float32, "dyn4_upd_sr", 3, 2),
+    (torch.float32, "dyn4_upd_sr_fp32read", 15, 1), (torch.float32, "dyn4_upd_sr_fp32read", 16, 2),
+    (torch.float32, "dyn4_proxy_la_upd_sr", 15, 1), (torch.float32, "dyn4_proxy_la_upd_sr", 16, 2)])
+def test_few_fp32_state_tiles_join_a_large_block_launch(dtype, m2, tiles, expect):
+    """A launch of their own beside 8,192 block tiles costs 5-6 us, more than one or two tiles of a wave take in a
+    specialised kernel."""
+    params = [torch.nn.Parameter(torch.zeros(n, device=H.DEVICE, dtype=dtype)) for n in [8192 * 1024] + [1000] * tiles]
+    opt = aw.QuantizedAdamW(params, m1_quant_scheme="nf4", m2_quant_scheme=m2, quant_rng_seed=1, optimized=True)
+    assert launches(params, opt) == expect
