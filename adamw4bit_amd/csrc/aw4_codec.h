@@ -129,9 +129,14 @@ struct Tables {
     float codebook[AW4_NUM_CODEBOOKS][16];
     UsrPair usr[AW4_NUM_CODEBOOKS][kPairs];  // per searchsorted index (update-SR)
     PairEntry pairs[AW4_NUM_CODEBOOKS][kPairs];
-    SsrEntry ssr[AW4_NUM_CODEBOOKS][kPairs];  // per searchsorted index (value-space SR)
     float2 dec[AW4_NUM_CODEBOOKS][256];  // code byte -> (level of low nibble, level of high nibble)
     LutEntry lut[AW4_NUM_LUTS][AW4_LUT_ENTRIES];
+};
+
+// What only the specialised kernels read, behind Tables in device memory.
+struct SpecTables {
+    SsrEntry ssr[AW4_NUM_CODEBOOKS][kPairs];  // per searchsorted index (value-space SR)
+    LinTable lin[AW4_NUM_LUTS];               // of every lookup-table id
 };
 
 // LDS views of the tables one moment needs.
@@ -141,7 +146,7 @@ struct MomentTables {
     const float2* dec;
     const LutEntry* lut;
     const UsrPair* usr;
-    const SsrEntry* ssr;
+    const SsrEntry* ssr;  // specialised kernels
     // LinEntry table (specialised kernels): magic, and the LDS address of an entry less 8 * the bits of
     // x + magic
     float lin_magic;

@@ -54,7 +54,7 @@
 // hipGetSymbolAddress (device_state) and uses only that.  (Only the main object holds them: the
 // second compile of this file, AW4_SCHED_ILP_TU below, emits kernels and nothing else.)
 #ifndef AW4_SCHED_ILP_TU
-static __device__ __align__(256) uint8_t g_tables_mem[sizeof(aw4::Tables) + AW4_NUM_LUTS * sizeof(aw4::LinTable)];
+static __device__ __align__(256) uint8_t g_tables_mem[sizeof(aw4::Tables) + sizeof(aw4::SpecTables)];
 // Launch tables of AW4_NOALLOC_TABLE_BYTES, and beyond them the header and the padding of every launch after
 // the first that such a table can split into: whether a call fits depends on its rows alone.
 constexpr size_t kNoallocGroupBytes = 1 << 17;
@@ -95,8 +95,8 @@ __host__ __device__ inline int lut_id_of(int rounding, int codebook, int flags) 
 // LDS layouts
 // ---------------------------------------------------------------------------
 
-// The LinTable of every lookup-table id, behind the other tables.
-__host__ __device__ inline const LinTable* lin_tables(const Tables* g) { return (const LinTable*)(g + 1); }
+// The specialised kernels' tables, behind those that every kernel reads.
+__host__ __device__ inline const SpecTables* spec_tables(const Tables* g) { return (const SpecTables*)(g + 1); }
 
 // Specialised kernels: the tables of the one codebook each moment uses.
 template <bool kUpd, bool kSsr>
@@ -134,9 +134,9 @@ struct LdsSlots {
             cb_v[w] = g->codebook[c][i16];
             usr_v[w] = *(const u32x4*)&g->usr[c][ip];
             pair_v[w] = *(const u32x4*)&g->pairs[c][ip];
-            if (kSsr) ssr_v[w] = *(const u32x4*)&g->ssr[c][ip];
+            if (kSsr) ssr_v[w] = *(const u32x4*)&spec_tables(g)->ssr[c][ip];
             dec_v[w] = *(const u32x2*)&g->dec[c][i];
-            const u32x4* e = (const u32x4*)lin_tables(g)[l].e;
+            const u32x4* e = (const u32x4*)spec_tables(g)->lin[l].e;
             lin_v[w] = e[i];
             lin_last[w] = e[kThreads];
         }
@@ -166,7 +166,7 @@ struct LdsAll {
         const int cbid = m.rounding == AW4_ROUND_FP32 ? 0 : m.codebook;
         return MomentTables{t.codebook[cbid], t.pairs[cbid], t.dec[cbid],
                             t.lut[m.rounding == AW4_ROUND_FP32 ? 0 : lut_id_of(m.rounding, cbid, m.flags)],
-                            t.usr[cbid], t.ssr[cbid], 0.0f, 0u};
+                            t.usr[cbid], nullptr, 0.0f, 0u};
     }
     __device__ f32x4* wave_m2_stage(int) { return nullptr; }
     __device__ void load(const Tables* g, const StepHeader*) {
@@ -244,11 +244,6 @@ __device__ __forceinline__ void step_body_inline(const InlineArgs& a) {
     const StepHeader* hdr =
         (const StepHeader*)((const char*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(InlineArgs, table));
     step_body<M1K, M2K, D>(hdr, a.tables);
-}
-
-template <int M1K, int M2K, int D>
-__global__ void __launch_bounds__(kThreads) step_kernel_inline(const InlineArgs a) {
-    step_body_inline<M1K, M2K, D>(a);
 }
 
 template <int M1K, int M2K, int D>
@@ -352,8 +347,6 @@ struct KernelVariant {
 #define AW4_VARIANT_4W(M1, M2, D) {M1, M2, D, (const void*)&step_kernel_4w<M1, M2, D>, nullptr}
 #define AW4_VARIANT_2W(M1, M2, D) {M1, M2, D, (const void*)&step_kernel_2w<M1, M2, D>, nullptr}
 #define AW4_VARIANT_3W(M1, M2, D) {M1, M2, D, (const void*)&step_kernel_3w<M1, M2, D>, nullptr}
-#define AW4_VARIANT_I(M1, M2, D) \
-    {M1, M2, D, (const void*)&step_kernel<M1, M2, D>, (const void*)&step_kernel_inline<M1, M2, D>}
 #define AW4_VARIANT_I4W(M1, M2, D) \
     {M1, M2, D, (const void*)&step_kernel_4w<M1, M2, D>, (const void*)&step_kernel_inline_4w<M1, M2, D>}
 // the max-ilp instances of the second object (their small-step instances stay in this one)
@@ -395,7 +388,6 @@ const KernelVariant kVariants[] = {
 #undef AW4_VARIANT_4W
 #undef AW4_VARIANT_2W
 #undef AW4_VARIANT_3W
-#undef AW4_VARIANT_I
 #undef AW4_VARIANT_I4W
 #undef AW4_VARIANT_ILP
 #undef AW4_VARIANT_ILP_3W
@@ -416,21 +408,20 @@ constexpr int kNumSpecialised = kResearchVariant;
 // Encoding nf4_sr is bound by its draws (26.7 us).
 constexpr int kCodecTiles = 4;
 
-// Encode tables of the codebook a moment uses, and the waves' scratch.
+// Encode tables of the codebook a moment uses, those its kind of rounding reads, and the waves' scratch.
+template <int KIND>
 struct LdsEncode {
     float cb[16];
-    UsrPair usr[kPairs];
-    PairEntry pairs[kPairs];
-    SsrEntry ssr[kPairs];
+    UsrPair usr[KIND == K_USR ? kPairs : 1];
+    PairEntry pairs[KIND != K_RTN ? kPairs : 1];
     LutEntry lut[AW4_LUT_ENTRIES];
     WaveScratch scratch[kWavesPerGroup];
 
     __device__ void load(const Tables* g, int codebook, int lut_id) {
         if (threadIdx.x < 16) cb[threadIdx.x] = g->codebook[codebook][threadIdx.x];
         if (threadIdx.x < kPairs) {
-            usr[threadIdx.x] = g->usr[codebook][threadIdx.x];
-            pairs[threadIdx.x] = g->pairs[codebook][threadIdx.x];
-            ssr[threadIdx.x] = g->ssr[codebook][threadIdx.x];
+            if constexpr (KIND == K_USR) usr[threadIdx.x] = g->usr[codebook][threadIdx.x];
+            if constexpr (KIND != K_RTN) pairs[threadIdx.x] = g->pairs[codebook][threadIdx.x];
         }
         if (threadIdx.x < AW4_LUT_ENTRIES) lut[threadIdx.x] = g->lut[lut_id][threadIdx.x];
         __syncthreads();
@@ -443,7 +434,7 @@ static_assert(AW4_LUT_ENTRIES <= kThreads, "one thread per lookup entry");
 template <int KIND>
 __global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restrict__ values, int64_t numel,
                                                             aw4_moment M, const Tables* __restrict__ tables) {
-    __shared__ LdsEncode lds;
+    __shared__ LdsEncode<KIND> lds;
     const int lane = threadIdx.x & 63;
     const int wslot = threadIdx.x >> 6;
     const int j = lane & 7, grp = lane >> 3;
@@ -464,7 +455,7 @@ __global__ void __launch_bounds__(kThreads) quantize_kernel(const float* __restr
     float next[16];
     if (tile < tiles) load(tile, next);
     lds.load(tables, M.codebook, lut_id_of(M.rounding, M.codebook, M.flags));
-    const MomentTables L{lds.cb, lds.pairs, nullptr, lds.lut, lds.usr, lds.ssr, 0.0f, 0u};
+    const MomentTables L{lds.cb, lds.pairs, nullptr, lds.lut, lds.usr, nullptr, 0.0f, 0u};
     while (tile < tiles) {
         float m[16];
 #pragma unroll
@@ -583,7 +574,7 @@ int rtn_code(const float* cb, float x, bool floor_zero) {
 
 struct HostTables {
     Tables t;
-    LinTable lin[AW4_NUM_LUTS];  // behind `t`, as in device memory
+    SpecTables spec;  // behind `t`, as in device memory
     bool ok = false;
     std::string error;
 };
@@ -720,7 +711,7 @@ const HostTables& host_tables() {
                 p.width_rcp = 1.0f / (w < 1e-12f ? 1e-12f : w);
                 p.lohi = (uint32_t)lo | ((uint32_t)hi << 8);
                 // (the 1e-12 floor of the width binds only where lo == hi: index 0, and 16, which no x <= 1 has)
-                SsrEntry& e = t.ssr[c][i];
+                SsrEntry& e = h.spec.ssr[c][i];
                 if (i > 0) {
                     e.a = p.a;
                     e.width = ldexpf(w < 1e-12f ? 1e-12f : w, -24);
@@ -741,13 +732,13 @@ const HostTables& host_tables() {
         if (ok) {
             const float* cb = t.codebook[AW4_CB_DYN4];
             ok = build_lut(t.lut[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, cb, h.error) &&
-                 build_linear_lut(h.lin[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, false, h.error);
+                 build_linear_lut(h.spec.lin[kLutRtnDyn4Floor], [cb](float x) { return rtn_code(cb, x, true); }, false, h.error);
         }
         for (int c = 0; c < AW4_NUM_CODEBOOKS && ok; ++c) {
             const float* cb = t.codebook[c];
             const bool is_signed = cb[0] < 0.0f;
-            ok = build_linear_lut(h.lin[kLutRtn[c]], [cb](float x) { return rtn_code(cb, x, false); }, is_signed, h.error) &&
-                 build_linear_lut(h.lin[kLutLevels[c]], [cb](float x) { return count_less(cb, x); }, is_signed, h.error);
+            ok = build_linear_lut(h.spec.lin[kLutRtn[c]], [cb](float x) { return rtn_code(cb, x, false); }, is_signed, h.error) &&
+                 build_linear_lut(h.spec.lin[kLutLevels[c]], [cb](float x) { return count_less(cb, x); }, is_signed, h.error);
         }
         h.ok = ok;
     });
@@ -799,8 +790,8 @@ int device_state(DeviceState** out) {
         void* stage = nullptr;
         AW4_HIP_CHECK(hipGetSymbolAddress(&tables, HIP_SYMBOL(g_tables_mem)));
         AW4_HIP_CHECK(hipGetSymbolAddress(&stage, HIP_SYMBOL(scratch)));
-        static_assert(offsetof(HostTables, lin) == sizeof(Tables), "one copy of both");
-        AW4_HIP_CHECK(hipMemcpy(tables, &ht.t, sizeof(Tables) + sizeof(ht.lin), hipMemcpyHostToDevice));
+        static_assert(offsetof(HostTables, spec) == sizeof(Tables), "one copy of both");
+        AW4_HIP_CHECK(hipMemcpy(tables, &ht.t, sizeof(Tables) + sizeof(SpecTables), hipMemcpyHostToDevice));
         ds.scratch = (uint8_t*)stage;
         ds.tables = (Tables*)tables;
     }
@@ -1195,8 +1186,8 @@ int fill_step_tables(const aw4_tensor* tensors, StepLaunch& sl, int num_cus, voi
         for (int w = 0; w < 2; ++w) {
             const int lut = w == 0 ? lg.lut1 : lg.lut2;
             if (lut < 0) continue;
-            h->lin_magic[w] = host_tables().lin[lut].magic;
-            h->lin_zero[w] = host_tables().lin[lut].zero;
+            h->lin_magic[w] = host_tables().spec.lin[lut].magic;
+            h->lin_zero[w] = host_tables().spec.lin[lut].zero;
         }
         h->total_tiles = acc;
         h->tiles_per_wave = tiles_per_wave;
