@@ -35,6 +35,7 @@ TENSOR_GRAD_UNSCALE = 0x10
 NUM_LUTS, LUT_HALF, LUT_EXP0 = 11, 89, 936
 NOALLOC_TABLE_BYTES = 1 << 20
 LUT_ENTRIES = 2 * LUT_HALF
+LINEAR_SLOTS = 514
 
 MOMENT = np.dtype([
     ("codes", "<u8"), ("scales", "<u8"), ("values", "<u8"), ("draws", "<u8"),
@@ -64,6 +65,7 @@ SIGNATURES = {
     "aw4_uniforms": (ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint64, ctypes.c_int64, ctypes.c_void_p,
                                     ctypes.c_void_p]),
     "aw4_encode_tables": (ctypes.c_int64, [ctypes.c_void_p, ctypes.c_int64]),
+    "aw4_linear_tables": (ctypes.c_int64, [ctypes.c_void_p, ctypes.c_int64]),
     "aw4_clip_coefficient": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_float, ctypes.c_void_p,
                                             ctypes.c_void_p, ctypes.c_void_p]),
     "aw4_unscale_clip_coefficient": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_float,
@@ -188,10 +190,25 @@ def uniforms(seed: int, offset: int, n: int, out_ptr: int, stream: int) -> None:
 
 
 def encode_tables() -> np.ndarray:
-    """The kernels' encode lookup tables, shape (NUM_LUTS, LUT_ENTRIES, 4) uint32 words
-    {threshold bits, base, level_lo bits, level_hi bits} (host only)."""
+    """The encode lookup tables of the generic kernels and the stand-alone encode, shape
+    (NUM_LUTS, LUT_ENTRIES, 4) uint32 words {threshold bits, base, level_lo bits, level_hi bits}
+    (host only)."""
     lib = library()
     size = check(lib.aw4_encode_tables(None, 0), "aw4_encode_tables")
     out = np.zeros(size // 4, dtype=np.uint32)
     check(lib.aw4_encode_tables(out.ctypes.data, size), "aw4_encode_tables")
     return out.reshape(NUM_LUTS, LUT_ENTRIES, 4)
+
+
+LINEAR_TABLE = np.dtype([("magic", "<f4"), ("count", "<i4"), ("zero", "<i4"), ("reserved", "<i4"),
+                         ("entries", [("threshold", "<f4"), ("base", "<u4")], (LINEAR_SLOTS,))])
+
+
+def linear_tables() -> np.ndarray:
+    """The specialised step kernels' lookup tables (NUM_LUTS of :data:`LINEAR_TABLE`, host only)."""
+    lib = library()
+    out = np.zeros(NUM_LUTS, dtype=LINEAR_TABLE)
+    size = check(lib.aw4_linear_tables(None, 0), "aw4_linear_tables")
+    assert size == out.nbytes
+    check(lib.aw4_linear_tables(out.ctypes.data, size), "aw4_linear_tables")
+    return out

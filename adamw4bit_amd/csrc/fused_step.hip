@@ -572,6 +572,8 @@ int rtn_code(const float* cb, float x, bool floor_zero) {
     return code;
 }
 
+static_assert(kLinSlots == AW4_LINEAR_SLOTS && sizeof(LinTable) == 16 + 8 * AW4_LINEAR_SLOTS, "aw4_linear_tables");
+
 struct HostTables {
     Tables t;
     SpecTables spec;  // behind `t`, as in device memory
@@ -1307,6 +1309,16 @@ int64_t aw4_encode_tables(void* out, int64_t bytes) {
     if (!out) return size;
     if (bytes < size) return set_error(AW4_EINVAL, "aw4_encode_tables: need %lld bytes", (long long)size);
     memcpy(out, ht.t.lut, (size_t)size);
+    return size;
+}
+
+int64_t aw4_linear_tables(void* out, int64_t bytes) {
+    const HostTables& ht = host_tables();
+    if (!ht.ok) return set_error(AW4_EINVAL, "encode tables: %s", ht.error.c_str());
+    const int64_t size = (int64_t)sizeof(ht.spec.lin);
+    if (!out) return size;
+    if (bytes < size) return set_error(AW4_EINVAL, "aw4_linear_tables: need %lld bytes", (long long)size);
+    memcpy(out, ht.spec.lin, (size_t)size);
     return size;
 }
 

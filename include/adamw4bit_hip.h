@@ -278,8 +278,8 @@ int aw4_unscale_clip_coefficient(const aw4_tensor* tensors, int32_t count, const
                                  float* norm_out, float* coef_out, float* found_inf_out, void* stream);
 
 /*
- * Host-only: copy the encode lookup tables the kernels use into `out`
- * (host memory, `bytes` long); returns the table size in bytes (call with
+ * Host-only: copy the encode lookup tables of the generic kernels and the
+ * stand-alone encode into `out` (host memory, `bytes` long); returns the table size in bytes (call with
  * out = 0 to query) or a negative error.  Layout: for each of AW4_NUM_LUTS
  * tables, AW4_LUT_ENTRIES entries {float threshold; uint32 base; float
  * level_lo; float level_hi}: a value x in bucket k (bucket function below)
@@ -297,6 +297,17 @@ int aw4_unscale_clip_coefficient(const aw4_tensor* tensors, int32_t count, const
 #define AW4_LUT_ENTRIES (2 * AW4_LUT_HALF)
 #define AW4_LUT_EXP0 936 /* (127 - 10) << 3: |x| < 2^-10 shares bucket 0 */
 int64_t aw4_encode_tables(void* out, int64_t bytes);
+
+/*
+ * Host-only, as aw4_encode_tables: the lookup tables of the specialised step
+ * kernels, the same AW4_NUM_LUTS tables in the same order.  Each is {float
+ * magic; int32 count; int32 zero; int32 reserved} and AW4_LINEAR_SLOTS entries
+ * {float threshold; uint32 base}, the first `count` of which are used: |x| <= 1
+ * (x >= 0 in a table with zero = 0) lies in entry bits(x + magic) - bits(magic)
+ * + zero, the sum rounded to fp32, and encodes to base + (x >= threshold).
+ */
+#define AW4_LINEAR_SLOTS 514
+int64_t aw4_linear_tables(void* out, int64_t bytes);
 
 #ifdef __cplusplus
 }

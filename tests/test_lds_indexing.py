@@ -5,7 +5,8 @@ bucket of x = m / s (from its bit pattern), the number of levels below x (`idx`,
 entry), the level neighbours of idx, the update-SR entry of idx, the decode entry of a code byte.
 Each restatement below follows the device code line for line (aw4_codec.h: lut_field,
 lut_bucket_unsigned / lut_bucket_signed, encode_block, update_sr_tables, encode_block_la; decode4)
-and the tables the library itself builds (aw4_encode_tables), and checks the index against the
+and the tables the library itself builds (aw4_encode_tables; the specialised kernels' linear ones are
+in test_linear_lookup), and checks the index against the
 size of the LDS array it reads, for every fp32 bit pattern class and for adversarial blocks
 (all zero, NaN and infinite values, huge and subnormal values, values on the levels).
 """

@@ -1,17 +1,22 @@
-"""The specialised kernels' lookup tables, restated: bucket of x = the step of the grid that fp32
-``x + magic`` rounds to, code or level count = base + (x >= thr).  Every bucket of [-1, 1] (or [0, 1])
-must hold at most one change, lie inside the LDS array, and give the exact count or code at and around
-every change and bucket edge."""
+"""The specialised kernels' lookup tables as the library builds them (aw4_linear_tables), read the way the
+kernels read them: entry = bits of the fp32 sum x + magic, less those of magic, plus the entry of 0; code or
+level count = base + (x >= threshold).  Every x of [-1, 1] (or [0, 1]) must lie inside the table and the LDS
+array, and give the exact count or code at and around every level, midpoint and bucket edge."""
 
 from __future__ import annotations
 
 import numpy as np
 import pytest
 
+from adamw4bit_amd import _lib
 from adamw4bit_amd import quantization as q
 
-SLOTS = 514
 F = np.float32
+
+
+@pytest.fixture(scope="module")
+def tables():
+    return _lib.linear_tables()
 
 
 def count_less(cb, x):
@@ -36,34 +41,71 @@ def around(values, ulps=6):
     return np.array(out, dtype=F)
 
 
-CASES = [(c, kind) for c in range(5) for kind in ("levels", "nearest")] + [(q.CB_DYN4, "floored")]
+def entry_of(table, x):
+    return (x + table["magic"]).view(np.int32) - table["magic"].reshape(1).view(np.int32) + table["zero"]
 
 
-@pytest.mark.parametrize("codebook,kind", CASES)
-def test_one_change_per_bucket(codebook, kind):
-    cb = np.array(q.CODEBOOK_VALUES[codebook], dtype=F)
-    signed = cb[0] < 0
-    f = (lambda x: count_less(cb, x)) if kind == "levels" else (lambda x: nearest(cb, x, kind == "floored"))
+def samples(cb, signed):
+    lo = -1 if signed else 0
     mids = (cb[1:].astype(np.float64) + cb[:-1]) / 2
-    for inv in (16, 32, 64, 128, 256, 512):
-        magic = F(1.5 * 2 ** 23 / inv)
-        zero = inv if signed else 0
-        slots = 2 * inv + 1 if signed else inv + 1
-        if slots > SLOTS:
-            pytest.fail("no bucket width holds one change each")
-        edges = (np.arange(-inv if signed else 0, inv) + 0.5) / inv
-        x = np.unique(np.concatenate([around(cb), around(mids), around(edges), around([0.0, 1.0]),
-                                      np.linspace(-1 if signed else 0, 1, 20001, dtype=F)]))
-        x = x[(x <= 1) & (x >= (-1 if signed else 0))]
-        bucket = (x + magic).view(np.int32) - magic.view(np.int32) + zero
-        assert bucket.min() == 0 and bucket.max() == slots - 1  # inside the table
-        value = f(x)
-        assert (np.diff(bucket) >= 0).all() and (np.diff(value) >= 0).all()
-        base = np.array([value[bucket == b].min() for b in range(slots)])
-        top = np.array([value[bucket == b].max() for b in range(slots)])
-        if (top - base <= 1).all():
-            break
-    # threshold: the first sampled x of the bucket with the higher value (the samples hold every change's
-    # two neighbours, so it is the first float too)
-    thr = np.array([x[(bucket == b) & (value == base[b] + 1)].min() if top[b] > base[b] else np.nan for b in range(slots)])
-    assert np.array_equal(base[bucket] + (x >= thr[bucket]), value)
+    edges = (np.arange(lo * 1024, 1024) + 0.5) / 1024  # every bucket edge of widths from 1/16 to 1/512, and between
+    edges = np.concatenate([edges, *((np.arange(lo * n, n) + 0.5) / n for n in (16, 32, 64, 128, 256, 512))])
+    x = np.unique(np.concatenate([around(cb), around(mids), around(edges, 2), around([0.0, 1.0, -1.0]),
+                                  F([1e-45, 1e-38, 1e-20]), np.linspace(lo, 1, 200001, dtype=F)]))
+    return x[(x <= 1) & (x >= lo)]
+
+
+# (lookup-table id, codebook, what it gives): round-to-nearest per codebook, dyn4 with the zero floor, level counts
+CASES = [(cb, cb, "nearest") for cb in range(5)] + [(5, q.CB_DYN4, "floored")] + [(6 + cb, cb, "levels") for cb in range(5)]
+
+
+@pytest.mark.parametrize("lut,codebook,kind", CASES)
+def test_table_gives_every_code_and_count(tables, lut, codebook, kind):
+    cb = np.array(q.CODEBOOK_VALUES[codebook], dtype=F)
+    signed = bool(cb[0] < 0)
+    t = tables[lut]
+    assert 0 < t["count"] <= _lib.LINEAR_SLOTS and (t["zero"] > 0) == signed and t["reserved"] == 0
+    x = samples(cb, signed)
+    entry = entry_of(t, x)
+    assert entry.min() == 0 and entry.max() == t["count"] - 1  # inside the table, and every end of it reached
+    assert (np.diff(entry) >= 0).all()
+    e = t["entries"][entry]
+    got = e["base"].astype(np.int64) + (x >= e["threshold"])
+    want = count_less(cb, x) if kind == "levels" else nearest(cb, x, kind == "floored")
+    wrong = np.flatnonzero(got != want)
+    assert not len(wrong), (x[wrong[:5]], got[wrong[:5]], want[wrong[:5]])
+
+
+def test_entries_keep_their_indexes_in_range(tables):
+    """Whatever x: base + 1 within the codes or level counts where a threshold can be reached, and the entries
+    behind the last one used are never read as codes beyond them either."""
+    for lut in range(_lib.NUM_LUTS):
+        t = tables[lut]
+        e = t["entries"]
+        top = 16 if lut >= 6 else 15
+        assert (e["base"].astype(np.int64) + np.isfinite(e["threshold"]) * (e["threshold"] <= 1)).max() <= top, lut
+
+
+def test_second_moments_lie_in_every_table(tables):
+    """Second moments are looked up by |x|, in tables of either kind."""
+    for lut in range(_lib.NUM_LUTS):
+        t = tables[lut]
+        x = samples(np.array(q.CODEBOOK_VALUES[q.CB_DYN4], dtype=F), False)
+        entry = entry_of(t, x)
+        assert entry.min() == t["zero"] and entry.max() == t["count"] - 1
+
+
+@pytest.mark.parametrize("field,change", [("magic", 2.0), ("zero", 1), ("count", -1), ("threshold", None)])
+def test_planted_fault_is_found(tables, field, change):
+    """The check above fails on a table with one field off (planted in a copy)."""
+    wrong = tables.copy()
+    t = wrong[6 + q.CB_NF4]
+    if field == "threshold":
+        k = int(np.flatnonzero(np.isfinite(t["entries"]["threshold"][:t["count"]]))[3])
+        t["entries"]["threshold"][k] = np.nextafter(t["entries"]["threshold"][k], F(4))
+    elif field == "magic":
+        t["magic"] *= F(change)
+    else:
+        t[field] += change
+    with pytest.raises((AssertionError, IndexError)):
+        test_table_gives_every_code_and_count(wrong, 6 + q.CB_NF4, q.CB_NF4, "levels")
