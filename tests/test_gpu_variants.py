@@ -1,6 +1,6 @@
 """Specialised kernels by dtype and scheme pair, at the sizes where a dispatch or a tile can go wrong:
 whole tiles, a last tile of a few blocks, a single 4-bit tensor of the smallest size, fp32-state tensors
-in the same launch, and a launch of more than one tile per wave.  Against the oracle, with the bars of
+in the same launch, and launches of two to twelve tiles per wave.  Against the oracle, with the bars of
 ``test_gpu_step`` (codes, scales and fp32 state bit-exact; parameters within the bars of ``gpu_helpers``)."""
 
 from __future__ import annotations
@@ -17,7 +17,7 @@ from tests.test_gpu_step import compare_pair, gpu_encode, log, moment_desc, run_
 
 pytestmark = pytest.mark.gpu
 
-# 4 whole tiles, 1 block past a whole tile, 1 block short of one, many tiles, fp32 state
+# 4 whole tiles, 1 block past a whole tile, 1 block short of one, many tiles (one per wave), fp32 state
 SHAPES = [(4096,), (33, 128), (71, 128), (1056, 2048), (4097,), (129,), (3,)]
 
 
@@ -194,3 +194,71 @@ def test_few_fp32_state_tiles_join_a_large_block_launch(dtype, m2, tiles, expect
     params = [torch.nn.Parameter(torch.zeros(n, device=H.DEVICE, dtype=dtype)) for n in [8192 * 1024] + [1000] * tiles]
     opt = aw.QuantizedAdamW(params, m1_quant_scheme="nf4", m2_quant_scheme=m2, quant_rng_seed=1, optimized=True)
     assert launches(params, opt) == expect
+
+
+# Every instance beside the recipes' fp32 and bf16 ones (those: test_gpu_step, test_gpu_fullsize).
+INSTANCES = ([("nf4", "dyn4_nz", True, torch.float16), ("nf4", "dyn4_upd_sr_fp32read", False, torch.float16),
+              ("nf4_sr", "dyn4_upd_sr_fp32read", False, torch.float16), ("nf4", "fp32", False, torch.float16),
+              ("nf4", "dyn4_upd_sr_fp32read", True, torch.float16)]
+             + [("sdyn4", "lin4_nz", False, dt) for dt in (torch.float32, torch.bfloat16, torch.float16)]
+             + [("nf4", m2, False, dt) for m2 in ("dyn4_upd_sr", "dyn4_proxy_la_upd_sr")
+                for dt in (torch.float32, torch.bfloat16, torch.float16)])
+
+
+def instance(m1, m2, eden):
+    return lambda ps: aw.QuantizedAdamW(ps, lr=1e-3, weight_decay=0.1, m1_quant_scheme=m1, m2_quant_scheme=m2,
+                                        use_eden_m2=eden, quant_rng_seed=3, optimized=True)
+
+
+@pytest.mark.parametrize("m1,m2,eden,dtype", INSTANCES)
+def test_two_tiles_per_wave_match_oracle(m1, m2, eden, dtype):
+    """32 tiles per CU, two for each wave, and a last tile of each tensor that is cut: the second tile's inputs are
+    loaded during the first one's encode."""
+    log(f"two tiles per wave {m1} / {m2} eden={eden} {dtype}")
+    out = run_pair(instance(m1, m2, eden), [(2048, 4096), (33, 128), (71, 128)], dtype, 2, seed=3, zero_block_frac=0.02,
+                   grad_fn=fp16_safe)
+    compare_pair(*out, f"two tiles {m1}/{m2} {dtype}", steps=2)
+
+
+def steps_of(make, shapes, dtype, shift, steps=2):
+    """Parameters and state after `steps` on the GPU, parameters and gradients `shift` values off a 16-byte boundary."""
+    params = []
+    gen = torch.Generator(device=H.DEVICE).manual_seed(1)
+    for s in shapes:
+        n = s[0] * s[1]
+        flat = torch.zeros(n + 8, device=H.DEVICE, dtype=dtype)
+        flat[shift:n + shift].normal_(0.0, 0.02, generator=gen)
+        params.append(torch.nn.Parameter(flat[shift:n + shift].view(s)))
+    opt = make(params)
+    for _ in range(steps):
+        for p in params:
+            n = p.numel()
+            flat = torch.zeros(n + 8, device=H.DEVICE, dtype=dtype)
+            # rows of magnitudes from e^-9 to e^-3, as heavy-tailed as an embedding's gradients
+            g = flat[shift:n + shift].normal_(generator=gen).view(p.shape)
+            g.mul_(torch.empty(p.shape[0], 1, device=H.DEVICE).uniform_(-9.0, -3.0, generator=gen).exp_().to(dtype))
+            p.grad = g
+        opt.step()
+        for p in params:
+            p.grad = None
+    out = []
+    for p in params:
+        st = opt.state[p]
+        out += [p.detach()] + [st[k] for k in ("m1", "m2", "m1_code", "m2_code") if k in st]
+        out += [st[k].absmax for k in ("m1_quant_state", "m2_quant_state") if st.get(k) is not None]
+    return out
+
+
+@pytest.mark.parametrize("m1,m2,eden,dtype,rows", [case + (8200,) for case in INSTANCES]
+                         + [case + (98400,) for case in INSTANCES if "upd_sr" in case[1]])
+def test_more_tiles_per_wave_match_generic_kernel(m1, m2, eden, dtype, rows):
+    """Three and four tiles per wave (128 tiles per CU), and twelve (1,536) of the kernels that take so many,
+    against the generic kernel, which steps the same tensors one value off their alignment: bit for bit."""
+    log(f"{rows} x 4096 {m1} / {m2} eden={eden} {dtype} against the generic kernel")
+    shapes = [(rows, 4096), (33, 128)]
+    got = steps_of(instance(m1, m2, eden), shapes, dtype, 0)
+    want = steps_of(instance(m1, m2, eden), shapes, dtype, 1)
+    assert len(got) == len(want)
+    for i, (a, b) in enumerate(zip(got, want)):
+        view = {4: torch.int32, 2: torch.int16, 1: torch.uint8}[a.element_size()]
+        assert torch.equal(a.contiguous().view(-1).view(view), b.contiguous().view(-1).view(view)), i
