@@ -411,7 +411,7 @@ struct BlockScales {
 // code its four quarters' table lookups, random numbers and roots overlap; with the tests for the general
 // rule between them (three branches a quarter) they ran one after the other: two Llama-3-8B layers under
 // ZIP-SR bf16 832 -> 822 us, the bf16 set with an nf4_sr head 1,652 -> 1,637 us, embedding and a layer in
-// fp32 1,870 -> 1,842 us (start's code on that box).  Kernels with a round-to-nearest second moment keep
+// fp32 1,870 -> 1,842 us.  Kernels with a round-to-nearest second moment keep
 // the loop below, which has one branch a quarter for them: as one stretch ZE-EDEN fp32 needed 107 VGPRs
 // instead of 96 and lost its fifth wave (GPT-2-small with clipping 414 -> 423 us).
 template <int KIND, bool kNonNeg, class Values>

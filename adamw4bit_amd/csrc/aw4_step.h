@@ -1020,7 +1020,7 @@ __device__ __forceinline__ void step_value_quads(const aw4_tensor& T, int64_t e0
 }
 
 // A launch of fp32-state tensors only (28 bytes a value in fp32, memory bound): no codec, so no LDS
-// tables, 84 VGPRs (six waves per SIMD), and each wave has its tile's 16 KB of loads in flight at once.
+// tables, 83 VGPRs (five waves per SIMD; 16-bit ones 79 and six), and each wave has its tile's 16 KB of loads in flight at once.
 // One tile per wave (no table to share between tiles).  A 201 MB fp32 set of odd sizes under ZIP-SR took
 // 69-71 us a step when these tiles went value by value inside the block kernel, 44 us here (4.5 TB/s);
 // a 306 MB fp16 one 357 -> 71 us, a 488 MB bf16 one 346 -> 98 us.

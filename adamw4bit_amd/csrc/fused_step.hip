@@ -1,4 +1,4 @@
-// Fused 4-bit AdamW step for MI355X (gfx950): one multi-tensor launch per optimizer step.
+// Fused 4-bit AdamW step for MI355X (gfx950): a multi-tensor launch for each kernel an optimizer step needs.
 //
 // Work decomposition
 //   * A 128-value block (one fp32 scale per moment) is owned by 8 lanes of a 64-lane
@@ -11,8 +11,8 @@
 //   * Tiles of all tensors form one index space; each wave takes up to 4 tiles (in grid
 //     order for the memory-bound kernels, consecutive ones for the update-SR kernels) and
 //     the grid covers all of them, so the hardware dispatcher keeps the tiles in flight a
-//     narrow moving window of memory.  One launch covers every parameter of the step,
-//     fp32-state tensors included.
+//     narrow moving window of memory.  fp32-state tensors join a launch of their dtype or
+//     take one of their own (plan_values).
 //   * Kernels are specialised on (m1 rounding kind, m2 rounding kind, parameter dtype);
 //     a launch table whose tensors share one such combination (every recipe) runs the
 //     specialised kernel, any other table the generic one.
@@ -209,17 +209,17 @@ step_kernel_4w(const StepHeader* __restrict__ hdr, const Tables* __restrict__ ta
 }
 
 // The same kernel held to 256 VGPRs, two waves per SIMD: the generic research instance (every
-// m2 kind, read back or lookahead, with run-time dtypes) needs 270 otherwise, one wave per SIMD;
-// the few registers it spills cost less than the second wave gains (pending lookahead 108 ->
-// 66 ms on the Llama-3-8B set).
+// m2 kind, read back or lookahead, with run-time dtypes) needed 270 otherwise, one wave per SIMD;
+// it takes 243, without spills, and the second wave took the pending lookahead from 108 to
+// 66 ms on the Llama-3-8B set.
 template <int M1K, int M2K, int D>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 step_kernel_2w(const StepHeader* __restrict__ hdr, const Tables* __restrict__ tables) {
     step_body<M1K, M2K, D>(hdr, tables);
 }
 
-// The same kernel held to 168 VGPRs, three waves per SIMD: the pending lookahead instance needs
-// 178 otherwise (two waves); six registers spill, and the third wave takes its step on the
+// The same kernel held to 168 VGPRs, three waves per SIMD: the pending lookahead instance needed
+// 178 otherwise (two waves); it takes 166, without spills, and the third wave took its step on the
 // Llama-3-8B set from 37.8 to 34.8 ms.
 template <int M1K, int M2K, int D>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
@@ -398,14 +398,16 @@ constexpr int kResearchVariant = kNumVariants - 2;  // generic, for read-back an
 constexpr int kNumSpecialised = kResearchVariant;
 
 // Stand-alone codec kernels.  They stream (encode reads 4 bytes and writes 0.53 a value, decode the
-// reverse), so a workgroup's LDS holds only the tables its one moment needs (8 KB of tables and the four
-// waves' scratch to encode, 2 KB to decode; all codebooks' tables are 36 KB and left three workgroups to
-// a CU), and the grid covers every tile at kCodecTiles per wave, which share the table fill.
-// Measured, nf4, us encode / decode of 2^24 values: 28 / 28 with all tables and a grid of eight
-// workgroups per CU, 14.9 / 13.4 so (5.1 / 5.7 TB/s); 2^27 values 112 / 124 us (5.4 / 4.9 TB/s).
+// reverse), so a workgroup's LDS holds only the tables its one moment needs (3 to 3.6 KB of tables and the
+// four waves' scratch, 8.3 KB, to encode, 2 KB to decode; all codebooks' tables are 36 KB and left three
+// workgroups to a CU), and the grid covers every tile at kCodecTiles per wave, which share the table fill.
 // Decode's stores are non-temporal, as the other kernels' are: dirty lines left in the L2s were written
-// back while the next launch waited (the pair, 2^24 values: 35.3 -> 27.6 us, 5.5 TB/s).
-// Encoding nf4_sr is bound by its draws (26.7 us).
+// back while the next launch waited.
+// Measured, nf4, us encode / decode: 2^24 values 26.5 / 27.6 with all tables, a grid of eight workgroups per
+// CU and plain stores, 13.6 / 12.1 so (5.6 / 6.3 TB/s); 2^27 values 140 / 160 and 111 / 89 us (5.5 / 6.8 TB/s).
+// A kernel that reads the decoded values next loses nothing: decode and a copy of 2^20, 2^22, 2^24 and 2^27
+// values 10.6, 30.7, 54.9 and 347 us before, 8.8, 16.1, 39.2 and 294 so.  Encoding nf4_sr is bound by its draws
+// (24.0 us of 2^24 values).
 constexpr int kCodecTiles = 4;
 
 // Encode tables of the codebook a moment uses, those its kind of rounding reads, and the waves' scratch.
@@ -966,7 +968,8 @@ void plan_values(const aw4_tensor* ts, const std::vector<int>& values, std::vect
 // Split a step's tensors into launches: tensors that share a specialised kernel and its
 // tables form one launch each; fp32-state tensors join one of their dtype or form their own
 // (plan_values); everything else (other scheme mixes, float64, mixed dtypes) runs in one launch of
-// the generic kernel.  A recipe's table is one launch.
+// the generic kernel.  A recipe's table is one launch, or two with many fp32-state tensors or some beside a
+// large launch; a step of several can fail after the first of them (AW4_ELAUNCHED).
 std::vector<LaunchGroup> plan_launches(const aw4_tensor* ts, int32_t count) {
     std::vector<LaunchGroup> groups;
     LaunchGroup generic, research;

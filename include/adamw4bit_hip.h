@@ -10,7 +10,7 @@
  * Reference interfaces replaced (nubank/adamw4bit, paths under src/adamw4bit/):
  *   aw4_fused_step   -> OptimizedBackend._step_parameter + _step_chunk
  *                       (_optimized.py:145-234) for EVERY parameter of one
- *                       optimizer.step() in a single launch; also the
+ *                       optimizer.step() in one call; also the
  *                       element arithmetic of the reference step
  *                       QuantizedAdamW.step (adamw.py:547-803) for the
  *                       scheme set it shares with the optimized path.
@@ -177,7 +177,9 @@ const char* aw4_last_error(void);
 /*
  * One fused AdamW step over `count` parameters on `stream` (a hipStream_t;
  * 0 = legacy default stream): one kernel launch per group of parameters that
- * share a kernel (one launch for a recipe's parameters).  `tensors` is a host
+ * share a kernel (one launch for a recipe's 4-bit parameters, which few
+ * fp32-state ones join; many, or some beside a large launch, take a second
+ * one, and the step can then fail with AW4_ELAUNCHED).  `tensors` is a host
  * array: a group of up to 11 parameters on the ZE-EDEN or ZIP-SR kernels
  * receives its rows in its launch's arguments, any other step's rows are
  * staged to device memory by the library (the call returns before the step
